@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <utility>
 #include <string>
 #include <vector>
@@ -228,7 +229,7 @@ bool same_spans(const cev_block& a, const cev_block& b) {
 
 struct Plan {
   std::vector<int32_t> tiles, segs, rows;
-  int32_t n_tiles = 0, n_segs = 0, tile_rows = 0, n_splits = 1, block_n = 0;
+  int32_t n_tiles = 0, n_segs = 0, tile_rows = 0, n_splits = 1, block_n = 0, fan_parts = 0, fan_subs = 0;
 };
 
 void push_seg(Plan& p, int32_t b, int32_t e, int32_t masked, int32_t s_cache) {
@@ -246,6 +247,90 @@ void push_seg(Plan& p, int32_t b, int32_t e, int32_t masked, int32_t s_cache) {
 // of an unmasked part plus a masked remainder: a short unmasked part would
 // cost a mostly empty key tile of its own.
 constexpr int32_t kMinFullLocal = 128;
+
+// Whether the small-launch kernel (a workgroup per 32 query slots, keys split
+// over its kFanWaves waves) runs this plan, by modelled times in us of both
+// forms.  The constants are fits to kernel traces of 60 launches (1-63
+// blocks of 8-96 rows after 0-32k keys and 1-16 bidirectional rows; 4 to
+// 256 workgroups of the 256-slot kernels), most within 15 % and none chosen
+// wrongly by more than 2 us:
+//   256-slot kernels: base + per-chunk time (it grows with the share f of
+//     busy slots) x chunks of the longest part x rounds of 256 workgroups, a
+//     gated epilogue where no merge carries it, and the merge by its bytes;
+//   this kernel: base + the larger of one workgroup's chain of sub-tile
+//     rounds and the CUs' total (a d = 256 or f32 workgroup fills a CU).
+// The new form has to win by 10 %.
+void choose_fan(const cev_attn_desc* d, Plan& p) {
+  const int g = d->n_q_heads / d->n_kv_heads;
+  const bool bf = d->dtype == CEV_BF16, wide = d->head_dim == 256;
+  const int32_t sub_rows = 32 / g;
+  int64_t rows = 0, n_subs = 0;
+  int32_t max_rows = 0, max_chunks = 0;
+  for (int32_t ti = 0; ti < p.n_tiles; ++ti) {
+    const int32_t* t = &p.tiles[(size_t)ti * 8];
+    rows += t[1];
+    n_subs += (t[1] + sub_rows - 1) / sub_rows;
+    max_rows = std::max(max_rows, t[1]);
+    max_chunks = std::max(max_chunks, t[4]);
+  }
+  // max_splits = 1 asks for one walk over every row's keys in stream order;
+  // beyond 16 workgroups a CU the 256-slot kernels fill the chip
+  if (p.n_tiles == 0 || d->max_splits == 1 || n_subs * d->n_kv_heads > 16 * kSplitTargetWorkgroups) return;
+  const auto merge_us = [&](int64_t parts) {
+    return parts > 1 ? 3.0 + 0.55e-6 * (double)(rows * d->n_q_heads * parts * cev_attn_record_bytes(d->dtype, d->head_dim)) : 0.0;
+  };
+  // 256-slot kernels
+  const double f = (double)max_rows / p.tile_rows;
+  const int64_t wgs = (int64_t)p.n_tiles * d->n_kv_heads * p.n_splits;
+  const double steps = (double)((wgs + kSplitTargetWorkgroups - 1) / kSplitTargetWorkgroups) * ((max_chunks + p.n_splits - 1) / p.n_splits);
+  double whole = merge_us(p.n_splits);
+  if (!bf)
+    whole += 8.0 + steps * (f > 0.5 ? 8.2 : 4.2);
+  else if (wide)
+    whole += 14.0 + steps * (0.9 + 0.9 * f) + (d->has_gate && p.n_splits == 1 ? 17.0 * f : 0.0);
+  else
+    whole += 9.5 + 4.0 * f + steps * (0.8 + 1.4 * f);
+  // this kernel: sub-tiles of every group of slots, whole or in n_splits parts
+  double best = 0.9 * whole;
+  for (const int64_t parts : {(int64_t)1, (int64_t)p.n_splits}) {
+    if (parts > 1 && p.n_splits == 1) break;
+    int64_t max_rounds = 0, sum_rounds = 0;
+    for (int32_t ti = 0; ti < p.n_tiles; ++ti) {
+      const int32_t* t = &p.tiles[(size_t)ti * 8];
+      for (int32_t r0 = t[0]; r0 < t[0] + t[1]; r0 += sub_rows) {
+        int32_t lo = INT32_MAX, hi = 0;  // local keys that the group's rows see
+        for (int32_t r = r0; r < std::min(r0 + sub_rows, t[0] + t[1]); ++r) {
+          const int32_t* rw = &p.rows[(size_t)r * 4];
+          if (rw[1] > rw[0]) lo = std::min(lo, rw[0]), hi = std::max(hi, rw[1]);
+          if (rw[2] >= 0) lo = std::min(lo, rw[2]), hi = std::max(hi, rw[2] + 1);
+        }
+        int64_t subs = 0;
+        for (int32_t si = t[2]; si < t[2] + t[3]; ++si) {
+          const int32_t* sg = &p.segs[(size_t)si * 4];
+          const int32_t b = sg[2] ? std::max(sg[0], lo) : sg[0], e = sg[2] ? std::min(sg[1], hi) : sg[1];
+          if (e > b) subs += (e - b + 31) / 32;
+        }
+        const int64_t rounds = (subs + kFanWaves * parts - 1) / (kFanWaves * parts);
+        max_rounds = std::max(max_rounds, rounds);
+        sum_rounds += rounds;
+      }
+    }
+    const double w = (double)(n_subs * d->n_kv_heads * parts), cus = kSplitTargetWorkgroups;
+    const double r = (double)max_rounds, avg = (double)sum_rounds / (double)n_subs;
+    double us = merge_us(parts);
+    if (!bf)
+      us += 6.0 + 5.2 * std::max(r, std::ceil(w / cus) * avg);
+    else if (wide)
+      us += 3.0 + std::max(10.0 + 2.0 * r, std::ceil(w / cus) * (10.0 + 2.0 * avg));
+    else
+      us += 6.0 + std::max(1.2 * r, w / cus * (1.25 * avg + 1.6));
+    if (us < best) {
+      best = us;
+      p.fan_parts = (int32_t)parts;
+      p.fan_subs = (max_rows + sub_rows - 1) / sub_rows;
+    }
+  }
+}
 
 int32_t build_plan(const cev_attn_desc* d, const cev_block* blocks, int32_t n, Plan& p) {
   int32_t rc = cev_check_attn_desc(d);
@@ -383,6 +468,7 @@ int32_t build_plan(const cev_attn_desc* d, const cev_block* blocks, int32_t n, P
     }
   }
   p.n_splits = (int32_t)split;
+  choose_fan(d, p);
   return CEV_OK;
 }
 
@@ -427,6 +513,8 @@ extern "C" int32_t cev_attn_plan_build(const cev_attn_desc* d, const cev_block* 
   h.bytes = (int32_t)need;
   h.n_splits = p.n_splits;
   h.block_n = p.block_n;
+  h.fan_parts = p.fan_parts;
+  h.fan_subs = p.fan_subs;
   int32_t* out = (int32_t*)plan;
   memcpy(out, &h, sizeof h);
   if (!p.tiles.empty()) memcpy(out + h.tiles_off, p.tiles.data(), 4 * p.tiles.size());

@@ -14,6 +14,9 @@
 // tile's keys are visited in key tiles of block_n keys (n_chunks of them);
 // with n_splits > 1 each tile's chunks are cut into n_splits contiguous
 // parts, one workgroup per (tile, part, kv head).
+// fan_parts > 0 asks for the small-launch kernel instead: one workgroup per
+// (tile, group of 32 query slots, part, kv head), fan_subs groups per tile
+// and fan_parts (1 or n_splits) parts.
 #pragma once
 #include <stdint.h>
 
@@ -46,7 +49,7 @@ struct cev_plan_header {
   int32_t t, s_cache, tile_rows, dtype;
   int32_t head_dim, n_q_heads, n_kv_heads, tiles_off;  // offsets in int32 units
   int32_t segs_off, rows_off, bytes, n_splits;
-  int32_t block_n, sig, reserved[2];
+  int32_t block_n, sig, fan_parts, fan_subs;
 };
 static_assert(sizeof(cev_plan_header) == 80, "plan header is 80 bytes");
 constexpr int32_t kPlanSigWord = 17;  // index of `sig` among the plan's int32 words
@@ -94,3 +97,7 @@ constexpr int kSplitMinChunks = 4;
 constexpr int kSplitMinChunksF32 = 2;
 constexpr int kSplitMergeChunks = 3;
 constexpr int kSplitMax = 256;
+// Waves of a small-launch workgroup.  Eight gave no shorter chain (two waves
+// then share a SIMD's issue slots) and one workgroup per CU instead of two
+// (8 x 61-77 bf16 tokens after 74 keys: 17.2 against 11.6 us).
+constexpr int kFanWaves = 4;

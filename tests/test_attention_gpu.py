@@ -16,7 +16,7 @@ import pytest
 
 import cev_hip
 from cev_hip import configs
-from bars import BF16_ABS, F32_ABS, assert_bf16, assert_f32, errors
+from bars import BF16_ABS, BF16_REL_EXACT, F32_ABS, assert_bf16, assert_f32, errors
 from helpers import GpuLayer, OracleLayer, default_table, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -319,6 +319,66 @@ def test_softmax_max_moves(gpu, orc, shape, max_splits):
         else:
             assert_f32(got, want, f"{shape} d={d}")
             assert_f32(got, want64, f"{shape} d={d} vs f64")
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,gated", [("bf16", 8, 8, 128, False), ("bf16", 16, 8, 128, True), ("bf16", 8, 1, 128, False),
+                                                  ("bf16", 16, 4, 256, True), ("f32", 16, 8, 128, False), ("f32", 8, 2, 128, True)])
+@pytest.mark.parametrize("case", ["one_key", "ragged", "tail", "split", "bidir", "scattered"])
+def test_small_launches_vs_oracle(gpu, orc, dtype, hq, hkv, d, gated, case):
+    """The small-launch kernel at its edges: one token without a prefix (one
+    key, three idle waves), groups cut inside blocks, a tail span, several
+    parts of the key stream with remainders, bidirectional rows with padded
+    ones, and more segments per tile than a wave has lanes."""
+    bf = dtype == "bf16"
+    cap = 0
+    if case == "one_key":
+        tab = cev_hip.BlockTable.from_rows(1, 1, 0, causal=True)
+    elif case == "ragged":
+        tab, _, _ = cev_hip.BlockTable.from_plans([(33, 33, 33)], [(0, n) for n in (1, 31, 32, 33, 7, 65)])
+    elif case == "tail":
+        tab, _, _ = cev_hip.BlockTable.from_plans([(129, 226, 129)], [(0, 5), (0, 40)])
+    elif case == "split":
+        tab, _, _ = cev_hip.BlockTable.from_plans([(1427, 1427, 1427)], [(0, 19), (0, 22)])
+    elif case == "bidir":
+        tab = cev_hip.BlockTable.from_rows(4, 43, 0, causal=False, lengths=[43, 17, 1, 0])
+    else:  # one-token questions in every other slot: one segment each
+        cap = 400
+        tab, _, _, _ = cev_hip.BlockTable.from_slots([(0, 70, 70)], [(0, 1, 100 + 2 * i) for i in range(130)], cap)
+    t, s = tab.t, tab.s_cache
+    rng = np.random.default_rng(17 * hq + d)
+    rnd = lambda *sh: rng.standard_normal(sh).astype(np.float32)  # noqa: E731
+    q, kn, vn, kc, vc, gate = rnd(t, hq, d), rnd(t, hkv, d), rnd(t, hkv, d), rnd(hkv, s, d), rnd(hkv, s, d), rnd(t, hq, d)
+    if bf:
+        q, kn, vn, kc, vc, gate = (orc.round_bf16(x) for x in (q, kn, vn, kc, vc, gate))
+    dv = lambda x: to_dev(x, bf, gpu)  # noqa: E731
+    qd, knd, vnd, kcd, vcd, gd = (dv(x) for x in (q, kn, vn, kc, vc, gate))
+    args = dict(k_cache=kcd if s else None, v_cache=vcd if s else None)
+    op = cev_hip.PackedAttention(qd, knd, tab, s_cache=s, has_gate=gated, gate=gd if gated else None, v_new=vnd, **args)
+    parts = int(op.plan.header()[18])
+    _say(f"small launch {case} {dtype} hq {hq} hkv {hkv} d {d}: tiles {op.plan.n_tiles}, parts {parts} of {op.plan.n_splits}")
+    assert parts >= 1 or case in ("one_key", "split"), "the planner should run this table on the small-launch kernel"
+    got = to_np(op(qd, knd, vnd, gate=gd if gated else None, **args))
+    mask = tab.to_dense_mask()
+    K, V = np.concatenate([kc, kn.transpose(1, 0, 2)], 1), np.concatenate([vc, vn.transpose(1, 0, 2)], 1)
+    # f64 over the same inputs; the parity bars of tests/bars.py, plus, for a
+    # gated bf16 layer, the gate's own op-by-op rounding: e^-g, 1 + e, the
+    # reciprocal, the output and the product are each rounded to bf16 (2^-9
+    # relative), so a row that sees one key (|v| up to 4.7) is up to
+    # 5 * 2^-9 |out| = 0.046 from exact whatever the attention did
+    g = hq // hkv
+    want = np.zeros((t, hq, d))
+    for h in range(hq):
+        z = q[:, h].astype(np.float64) @ K[h // g].astype(np.float64).T / np.sqrt(d) + mask
+        z = np.exp(z - z.max(1, keepdims=True))
+        want[:, h] = z / z.sum(1, keepdims=True) @ V[h // g].astype(np.float64)
+    if gated:
+        want /= 1.0 + np.exp(-gate.astype(np.float64))
+    if bf:
+        own = 5 * 2.0**-9 * np.abs(want) if gated else 0.0
+        err = np.abs(got - want) - own
+        assert np.isfinite(got).all() and err.max() <= BF16_ABS and err.max() <= BF16_REL_EXACT * np.abs(want).max(), err.max()
+    else:
+        assert_f32(got, want, f"{case} d={d}")
 
 
 def test_packed_equals_each_block_alone_on_gpu(gpu):
