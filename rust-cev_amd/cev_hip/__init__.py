@@ -17,8 +17,8 @@ from typing import Optional, Sequence
 import numpy as np
 
 from . import synth  # noqa: F401  (re-exported)
-from ._abi import (CEV_BF16, CEV_F32, CEV_LINEAR_WORKSPACE_BYTES, CEV_MAX_SPANS, AttnDesc, Block, CevError, GdnDesc, QkNormDesc, Span,
-                   check, lib)
+from ._abi import (CEV_BF16, CEV_ERR_SPACE, CEV_F32, CEV_LINEAR_WORKSPACE_BYTES, CEV_MAX_SPANS, AttnDesc, Block, CevError, GdnDesc, Span,
+                   calls, check, lib)
 
 __all__ = [
     "GatedDeltaNet",
@@ -60,14 +60,36 @@ class BlockTable:
     """A list of cev_block rows: which keys each packed query row sees."""
 
     def __init__(self, blocks: Sequence[Block], t: int, s_cache: int):
-        self.blocks = list(blocks)
+        self._blocks = list(blocks)
+        self._built = None
         self.t = int(t)
         self.s_cache = int(s_cache)
 
+    @classmethod
+    def _from_array(cls, arr, n: int, t: int, s_cache: int):
+        """A table over the first n blocks of a ctypes array that a builder
+        filled; the Python list is made only when someone asks for it."""
+        tab = cls((), t, s_cache)
+        tab._blocks, tab._built = None, (arr, n)
+        return tab
+
+    @property
+    def blocks(self):
+        if self._blocks is None:  # from here on the list is the table
+            arr, n = self._built
+            self._blocks, self._built = [arr[i] for i in range(n)], None
+        return self._blocks
+
+    @blocks.setter
+    def blocks(self, value):
+        self._blocks, self._built = list(value), None
+
     def __len__(self):
-        return len(self.blocks)
+        return self._built[1] if self._blocks is None else len(self._blocks)
 
     def array(self):
+        if self._blocks is None:
+            return self._built[0]
         arr = (Block * max(1, len(self.blocks)))()
         for i, b in enumerate(self.blocks):
             arr[i] = b
@@ -103,7 +125,7 @@ class BlockTable:
         check(L.cev_table_from_plans(n_pl, past, pre, ts, len(items), ip, il, blocks, nb.value, C.byref(nb), pos, nt.value,
                                      C.byref(nt), gather))
         s_cache = int(sum(p[0] for p in plans))
-        tab = cls([blocks[i] for i in range(nb.value)], nt.value, s_cache)
+        tab = cls._from_array(blocks, nb.value, nt.value, s_cache)
         return tab, np.frombuffer(pos, np.int32)[: nt.value].copy(), np.frombuffer(gather, np.int32)[: len(items)].copy()
 
     @classmethod
@@ -124,7 +146,7 @@ class BlockTable:
         gather = (C.c_int32 * max(1, len(items)))()
         check(L.cev_table_from_slots(len(plans), kb, pre, ts, len(items), ip, il, isl, int(capacity), blocks, nb.value, C.byref(nb), pos,
                                      slots, nt.value, C.byref(nt), gather))
-        tab = cls([blocks[i] for i in range(nb.value)], nt.value, int(capacity))
+        tab = cls._from_array(blocks, nb.value, nt.value, int(capacity))
         as_np = lambda x, n: np.frombuffer(x, np.int32)[:n].copy()  # noqa: E731
         return tab, as_np(pos, nt.value), as_np(slots, nt.value), as_np(gather, len(items))
 
@@ -134,7 +156,7 @@ class BlockTable:
         blocks = (Block * max(1, b))()
         ln = None if lengths is None else (C.c_int32 * max(1, b))(*[int(x) for x in lengths])
         check(lib().cev_table_from_rows(b, t, past, 1 if causal else 0, ln, blocks, b))
-        return cls([blocks[i] for i in range(b)], b * t, past)
+        return cls._from_array(blocks, b, b * t, past)
 
     @classmethod
     def from_segment_ids(cls, seg, past: int = 0):
@@ -180,25 +202,58 @@ def attn_desc(dtype: int, hq: int, hkv: int, d: int, t: int, s_cache: int, has_g
     return desc
 
 
+def upload_async(arrays, device):
+    """Host arrays as device tensors (of their dtypes) through one pinned
+    buffer and one copy on the current stream, without waiting for it: for
+    arrays that the caller uses on this stream only.  A pageable copy makes
+    the host wait for everything queued on the stream before it.  Refused
+    under capture, where the copy would read the buffer again on replay."""
+    torch = _torch()
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("host arrays cannot be uploaded while the stream is being captured")
+    arrays = [np.ascontiguousarray(a) for a in arrays]
+    offs, total = [], 0
+    for a in arrays:
+        offs.append(total)
+        total += (a.nbytes + 15) // 16 * 16
+    host = torch.empty(max(16, total), dtype=torch.uint8, pin_memory=True)
+    view = host.numpy()
+    for a, o in zip(arrays, offs):
+        view[o: o + a.nbytes] = a.reshape(-1).view(np.uint8)
+    dev = host.to(device, non_blocking=True)  # the pinned allocator keeps the buffer until the copy has run
+    kinds = {"int32": torch.int32, "uint8": torch.uint8}
+    return [dev[o: o + a.nbytes].view(kinds[a.dtype.name]).view(a.shape) for a, o in zip(arrays, offs)]
+
+
 class AttnPlan:
     """A table compiled for one descriptor: host bytes plus a device copy."""
 
     def __init__(self, desc: AttnDesc, table: BlockTable, device=None):
         L = lib()
         arr = table.array()
-        size = C.c_size_t()
-        check(L.cev_attn_plan_size(C.byref(desc), arr, len(table), C.byref(size)))
-        raw = np.zeros(size.value + 16, np.uint8)
-        off = (-raw.ctypes.data) % 16
-        self.host = raw[off: off + size.value]
-        check(L.cev_attn_plan_build(C.byref(desc), arr, len(table), C.c_void_p(self.host.ctypes.data), size.value))
+        # room for the usual plan (16 bytes a row, a few segments a block);
+        # the exact size is asked for only when that was too small
+        size = min(1024 + 16 * max(0, int(desc.t)) + 256 * len(table), 1 << 24)
+        while True:
+            raw = np.empty(size + 16, np.uint8)
+            off = (-raw.ctypes.data) % 16
+            base = raw.ctypes.data + off
+            rc = L.cev_attn_plan_build(C.byref(desc), arr, len(table), C.c_void_p(base), size)
+            if rc != CEV_ERR_SPACE:
+                break
+            need = C.c_size_t()
+            check(L.cev_attn_plan_size(C.byref(desc), arr, len(table), C.byref(need)))
+            size = need.value
+        check(rc)
+        nbytes = int(raw[off: off + 80].view(np.int32)[14])
+        self.host = raw[off: off + nbytes]
         hdr = self.header()
         self.n_tiles = int(hdr[2])
         self.n_segs = int(hdr[3])
         self.tile_rows = int(hdr[6])
         self.n_splits = int(hdr[15])
         self.block_n = int(hdr[16])
-        self.nbytes = size.value
+        self.nbytes = nbytes
         ws = C.c_size_t()
         check(L.cev_attn_workspace_size(C.c_void_p(self.host.ctypes.data), C.byref(ws)))
         self.workspace_bytes = ws.value
@@ -236,6 +291,19 @@ class PackedAttention:
 
     def __init__(self, q, k_new, table: BlockTable, k_cache=None, s_cache: int = 0, has_gate: bool = False,
                  scale: Optional[float] = None, out=None, gate=None, v_new=None, v_cache=None, max_splits: int = 0):
+        self._setup(q, k_new, table, k_cache, s_cache, has_gate, scale, out, gate, v_new, v_cache, max_splits)
+        self.plan = AttnPlan(self.desc, table, device=q.device)
+
+    @classmethod
+    def _host_planned(cls, q, k_new, table, k_cache, s_cache, out, v_new, v_cache, max_splits):
+        """The same with the plan on the host only: the caller places
+        plan.dev and plan.workspace."""
+        op = cls.__new__(cls)
+        op._setup(q, k_new, table, k_cache, s_cache, False, None, out, None, v_new, v_cache, max_splits)
+        op.plan = AttnPlan(op.desc, table)
+        return op
+
+    def _setup(self, q, k_new, table, k_cache, s_cache, has_gate, scale, out, gate, v_new, v_cache, max_splits):
         t, hq, d = q.shape
         hkv = k_new.shape[1]
         if table.t != t or table.s_cache != s_cache:
@@ -245,7 +313,6 @@ class PackedAttention:
         self.desc.max_splits = int(max_splits)
         self._set_strides(q, k_new, v_new if v_new is not None else k_new, k_cache, v_cache if v_cache is not None else k_cache,
                           out if out is not None else q, gate)
-        self.plan = AttnPlan(self.desc, table, device=q.device)
 
     def _set_strides(self, q, kn, vn, kc, vc, out, gate):
         D = self.desc
@@ -263,13 +330,11 @@ class PackedAttention:
             D.g_stride_t, D.g_stride_h = gate.stride(0), gate.stride(1)
 
     def __call__(self, q, k_new, v_new, k_cache=None, v_cache=None, gate=None, out=None, stream=None):
-        torch = _torch()
         if out is None:
-            out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        self._set_strides(q, k_new, v_new, k_cache, v_cache, out, gate)
-        check(lib().cev_packed_attention(C.byref(self.desc), C.c_void_p(self.plan.host.ctypes.data), _ptr(self.plan.dev), _ptr(q),
-                                         _ptr(k_cache), _ptr(v_cache), _ptr(k_new), _ptr(v_new), _ptr(gate), _ptr(out),
-                                         _ptr(self.plan.workspace), self.plan.workspace_bytes, _stream_ptr(stream)))
+            out = _torch().empty(q.shape, dtype=q.dtype, device=q.device)
+        plan = self.plan
+        calls().attention(self.desc, plan.host, plan.dev, q, k_new, v_new, k_cache, v_cache, gate, out, plan.workspace,
+                          plan.workspace_bytes, stream)
         return out
 
 
@@ -318,27 +383,13 @@ class Rotary:
 def qknorm_rope(q_in, k_in, w_q, w_k, pos, rot: Rotary, eps: float, plus_one: bool = False, q_out=None, k_out=None, stream=None):
     """RMSNorm + RoPE of q (t, hq, d) and k (t, hkv, d) views (qwen3.rs:193-196,
     qwen35.rs:529-539).  q_in may be a strided view of a gated q_proj output."""
-    torch = _torch()
-    t, hq, d = q_in.shape
-    hkv = k_in.shape[1]
-    code = _dtype_code(q_in)
     if q_out is None:
-        q_out = torch.empty((t, hq, d), dtype=q_in.dtype, device=q_in.device)
+        q_out = _torch().empty(tuple(q_in.shape), dtype=q_in.dtype, device=q_in.device)
     if k_out is None:
-        k_out = torch.empty((t, hkv, d), dtype=k_in.dtype, device=k_in.device)
-    desc = QkNormDesc()
-    check(lib().cev_qknorm_desc_init(C.byref(desc), code, hq, hkv, d, t, rot.rotary_dim, rot.n_pos, 1 if plus_one else 0, float(eps), 0))
-    for t_ in (q_in, k_in, q_out, k_out):
-        if t_.stride(-1) != 1:
-            raise CevError(-2, "last dimension must be contiguous")
-    desc.qi_stride_t, desc.qi_stride_h = q_in.stride(0), q_in.stride(1)
-    desc.ki_stride_t, desc.ki_stride_h = k_in.stride(0), k_in.stride(1)
-    desc.qo_stride_t, desc.qo_stride_h = q_out.stride(0), q_out.stride(1)
-    desc.ko_stride_t, desc.ko_stride_h = k_out.stride(0), k_out.stride(1)
-    if pos.dtype != torch.int32:
-        raise CevError(-1, "positions must be int32")
-    check(lib().cev_qknorm_rope(C.byref(desc), _ptr(q_in), _ptr(k_in), _ptr(w_q), _ptr(w_k), _ptr(pos), _ptr(rot.cos), _ptr(rot.sin),
-                                _ptr(q_out), _ptr(k_out), _stream_ptr(stream)))
+        t, _, d = q_in.shape
+        k_out = _torch().empty((t, k_in.shape[1], d), dtype=k_in.dtype, device=k_in.device)
+    calls().qknorm_rope(q_in, k_in, w_q, w_k, pos, rot.cos, rot.sin, rot.rotary_dim, rot.n_pos, eps, plus_one, q_out, k_out, None, None,
+                        None, 0, stream)
     return q_out, k_out
 
 
@@ -348,24 +399,8 @@ def qknorm_rope_kv(q_in, k_in, v_in, w_q, w_k, pos, rot: Rotary, eps: float, q_o
     (normalised, rotated) and v (copied) of token i land in row slots[i] of
     k_out / v_out (row i without slots), e.g. (t_or_capacity, hkv, d) views
     of head-major caches."""
-    torch = _torch()
-    t, hq, d = q_in.shape
-    hkv = k_in.shape[1]
-    code = _dtype_code(q_in)
-    desc = QkNormDesc()
-    check(lib().cev_qknorm_desc_init(C.byref(desc), code, hq, hkv, d, t, rot.rotary_dim, rot.n_pos, 1 if plus_one else 0, float(eps), 0))
-    for t_ in (q_in, k_in, v_in, q_out, k_out, v_out):
-        if t_.stride(-1) != 1:
-            raise CevError(-2, "last dimension must be contiguous")
-    desc.qi_stride_t, desc.qi_stride_h = q_in.stride(0), q_in.stride(1)
-    desc.ki_stride_t, desc.ki_stride_h = k_in.stride(0), k_in.stride(1)
-    desc.qo_stride_t, desc.qo_stride_h = q_out.stride(0), q_out.stride(1)
-    desc.ko_stride_t, desc.ko_stride_h = k_out.stride(0), k_out.stride(1)
-    if pos.dtype != torch.int32 or (slots is not None and slots.dtype != torch.int32):
-        raise CevError(-1, "positions and slots must be int32")
-    check(lib().cev_qknorm_rope_kv(C.byref(desc), _ptr(q_in), _ptr(k_in), _ptr(v_in), v_in.stride(0), v_in.stride(1), _ptr(w_q),
-                                   _ptr(w_k), _ptr(pos), _ptr(rot.cos), _ptr(rot.sin), _ptr(slots), int(n_slots), _ptr(q_out),
-                                   _ptr(k_out), _ptr(v_out), v_out.stride(0), v_out.stride(1), _stream_ptr(stream)))
+    calls().qknorm_rope(q_in, k_in, w_q, w_k, pos, rot.cos, rot.sin, rot.rotary_dim, rot.n_pos, eps, plus_one, q_out, k_out, v_in, v_out,
+                        slots, n_slots, stream)
     return q_out, k_out, v_out
 
 
@@ -376,33 +411,22 @@ def rms_norm(x, w, eps: float, h=None, x_out=None, y=None, plus_one: bool = Fals
     and normalised.  sequential=True sums the squares in element order
     (cev_rms_norm_seq, candle's CPU order bit for bit) instead of tree order.
     Returns y."""
-    torch = _torch()
-    rows, hidden = x.shape
     if y is None:
-        y = torch.empty((rows, hidden), dtype=x.dtype, device=x.device)
+        rows, hidden = x.shape
+        y = _torch().empty((rows, hidden), dtype=x.dtype, device=x.device)
     if h is not None and x_out is None:
         x_out = x
-    for t_ in (x, y, w) + ((h, x_out) if h is not None else ()):
-        if t_.stride(-1) != 1 or t_.dtype != x.dtype:
-            raise CevError(-2, "rms_norm: tensors must share the dtype and have a contiguous last dim")
-    fn = lib().cev_rms_norm_seq if sequential else lib().cev_rms_norm
-    check(fn(_dtype_code(x), rows, hidden, _ptr(x), x.stride(0), _ptr(h), h.stride(0) if h is not None else 0,
-                             _ptr(x_out), x_out.stride(0) if x_out is not None else 0, _ptr(w), float(eps), 1 if plus_one else 0,
-                             _ptr(y), y.stride(0), _stream_ptr(stream)))
+    calls().rms_norm(x, w, eps, h, x_out, y, plus_one, stream, sequential)
     return y
 
 
 def swiglu(gate, up, out=None, stream=None):
     """silu(gate) * up in the model dtype (Mlp::forward, qwen3.rs:230-233);
     gate and up are (rows, inter) views sharing a row stride."""
-    torch = _torch()
-    rows, inter = gate.shape
-    if up.shape != gate.shape or up.stride(0) != gate.stride(0):
-        raise CevError(-1, "swiglu: gate and up must have the same shape and row stride")
     if out is None:
-        out = torch.empty((rows, inter), dtype=gate.dtype, device=gate.device)
-    check(lib().cev_swiglu(_dtype_code(gate), rows, inter, _ptr(gate), _ptr(up), gate.stride(0), _ptr(out), out.stride(0),
-                           _stream_ptr(stream)))
+        rows, inter = gate.shape
+        out = _torch().empty((rows, inter), dtype=gate.dtype, device=gate.device)
+    calls().swiglu(gate, up, out, stream)
     return out
 
 
@@ -465,23 +489,12 @@ def linear(x, w, out=None, alpha: float = 1.0, out_dtype=None, blas: Optional[Bl
     """out = out_dtype(alpha * x @ w.T) for x (m, k), w (n, k): candle's bias-free
     Linear::forward (qwen3.rs:175-178, :229-233), the code head (engine.rs:463)
     and the d3 readout (hybrid.rs:657, alpha = 1 / temperature)."""
-    torch = _torch()
-    m, k = x.shape
-    n = w.shape[0]
-    code = _dtype_code(x)
-    if w.dtype != x.dtype or w.shape[1] != k:
-        raise CevError(-1, "linear: w must be (n, k) in x's dtype")
-    out_dtype = x.dtype if out_dtype is None else out_dtype
+    m = x.shape[0]
     if out is None:
-        out = torch.empty((m, n), dtype=out_dtype, device=x.device)
-    for t_ in (x, w, out):
-        if t_.stride(-1) != 1:
-            raise CevError(-2, "linear: last dimension must be contiguous")
-    blas = Blas.on(x.device) if (blas is None and m > 8) else blas
-    ws = blas.workspace if blas is not None else None
-    check(lib().cev_linear(blas.handle if blas is not None else None, code, _dtype_code(out), m, n, k, _ptr(x), x.stride(0), _ptr(w),
-                           w.stride(0), float(alpha), _ptr(out), out.stride(0), _ptr(ws), ws.numel() if ws is not None else 0,
-                           _stream_ptr(stream)))
+        out = _torch().empty((m, w.shape[0]), dtype=x.dtype if out_dtype is None else out_dtype, device=x.device)
+    if blas is None and m > 8:
+        blas = Blas.on(x.device)
+    calls().linear(x, w, out, alpha, None if blas is None else blas.handle.value, None if blas is None else blas.workspace, stream)
     return out
 
 
@@ -489,16 +502,11 @@ def gather_rows(table, ids=None, out=None, out_dtype=None, stream=None):
     """out[i] = table[ids[i]] converted to out_dtype (Embedding rows,
     qwen3.rs:288-293; index_select of answer rows, qwen3.rs:399;
     to_dtype(F32), qwen3.rs:400, with ids None)."""
-    torch = _torch()
-    rows, width = table.shape
-    n = rows if ids is None else ids.shape[0]
-    if ids is not None and (ids.dtype != torch.int32 or not ids.is_contiguous()):
-        raise CevError(-1, "gather_rows: ids must be contiguous int32")
-    out_dtype = table.dtype if out_dtype is None else out_dtype
     if out is None:
-        out = torch.empty((n, width), dtype=out_dtype, device=table.device)
-    check(lib().cev_gather_rows(_dtype_code(table), _dtype_code(out), n, width, _ptr(table), table.stride(0), rows, _ptr(ids), _ptr(out),
-                                out.stride(0), _stream_ptr(stream)))
+        rows, width = table.shape
+        n = rows if ids is None else ids.shape[0]
+        out = _torch().empty((n, width), dtype=table.dtype if out_dtype is None else out_dtype, device=table.device)
+    calls().gather_rows(table, ids, out, stream)
     return out
 
 
@@ -638,31 +646,11 @@ class GatedDeltaNet:
                  s_out=None, stream=None):
         torch = _torch()
         B, T, nk, nv, dk, dv, K = self.shape
-        D = self.desc
-        for name, x in (("mixed", mixed), ("z", z), ("b", b), ("a", a)):
-            if x.stride(-1) != 1 or x.dtype != self.dtype:
-                raise ValueError(f"{name} must be {self.dtype} with unit channel stride")
-        D.mixed_stride_b, D.mixed_stride_t = mixed.stride(0), mixed.stride(1)
-        D.z_stride_b, D.z_stride_t = z.stride(0), z.stride(1)
-        if a.stride() != b.stride():
-            raise ValueError("a and b must share strides")
-        D.ab_stride_b, D.ab_stride_t = a.stride(0), a.stride(1)
-        if conv_in is not None:
-            if conv_in.stride(1) != K - 1 or conv_in.stride(2) != 1:
-                raise ValueError("conv_in must be (B, conv_dim, K-1) with contiguous rows")
-            D.conv_in_stride_b = conv_in.stride(0)
-        if s_in is not None:
-            if s_in.dtype != torch.float32 or tuple(s_in.stride()[1:]) != (dk * dv, dv, 1):
-                raise ValueError("s_in must be f32 (B, nv, dk, dv) with contiguous heads")
-            D.s_in_stride_b = s_in.stride(0)
         if y is None:
             y = torch.empty((B, T, nv * dv), dtype=self.dtype, device=mixed.device)
-        D.y_stride_b, D.y_stride_t = y.stride(0), y.stride(1)
         if conv_out is None:
             conv_out = torch.empty((B, self.conv_dim, K - 1), dtype=self.dtype, device=mixed.device)
         if s_out is None:
             s_out = torch.empty((B, nv, dk, dv), dtype=torch.float32, device=mixed.device)
-        check(lib().cev_gdn_forward(C.byref(D), _ptr(mixed), _ptr(z), _ptr(b), _ptr(a), _ptr(conv_w), _ptr(neg_a), _ptr(dt_bias),
-                                    _ptr(norm_w), _ptr(conv_in), _ptr(s_in), _ptr(y), _ptr(conv_out), _ptr(s_out),
-                                    _ptr(self.workspace), self.workspace.numel(), _stream_ptr(stream)))
+        calls().gdn(self.desc, mixed, z, b, a, conv_w, neg_a, dt_bias, norm_w, conv_in, s_in, y, conv_out, s_out, self.workspace, stream)
         return y, conv_out, s_out

@@ -146,6 +146,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_calls = None
 
 
 class CevError(RuntimeError):
@@ -170,6 +171,27 @@ def lib():
             fn.argtypes = args
         _lib = L
     return _lib
+
+
+def calls():
+    """The native launch calls (csrc/py_calls.cpp), bound to the loaded
+    library: they read tensors in C++ instead of through ctypes."""
+    global _calls
+    if _calls is None:
+        import importlib.machinery
+        import importlib.util
+
+        import torch  # noqa: F401  (the module links against its libraries)
+        path = os.path.join(_PKG, "build", "_cev_calls.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
+        loader = importlib.machinery.ExtensionFileLoader("_cev_calls", path)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_cev_calls", path, loader=loader))
+        loader.exec_module(mod)
+        L = lib()
+        mod.bind(CevError, {name: C.cast(getattr(L, name), P).value for name in SIGNATURES})
+        _calls = mod
+    return _calls
 
 
 def check(rc: int) -> None:

@@ -20,7 +20,7 @@ from __future__ import annotations
 
 import numpy as np
 
-from . import (BlockTable, PackedAttention, Rotary, gather_rows, linear, qknorm_rope_kv, rms_norm, swiglu)
+from . import (BlockTable, PackedAttention, Rotary, gather_rows, linear, qknorm_rope_kv, rms_norm, swiglu, upload_async)
 
 
 class Qwen3Stack:
@@ -70,9 +70,7 @@ class Qwen3Stack:
         if table.t != t or table.s_cache != self.capacity:
             raise ValueError(f"table is for t={table.t}, s_cache={table.s_cache}; pass has t={t}, capacity={self.capacity}")
         H, hq, hkv, d = w.hidden, w.hq, w.hkv, w.d
-        i32 = lambda a: torch.as_tensor(np.ascontiguousarray(a, np.int32), device=self.device)  # noqa: E731
-        ids, pos_d, slots_d = i32(tokens), i32(pos), i32(slots)
-        x = gather_rows(self.embed, ids)
+        x = torch.empty((t, H), dtype=self.dtype, device=self.device)
         y = torch.empty_like(x)
         q = torch.empty((t, hq, d), dtype=self.dtype, device=self.device)
         o = torch.empty((t, hq, d), dtype=self.dtype, device=self.device)
@@ -82,8 +80,15 @@ class Qwen3Stack:
         h = torch.empty_like(x)
         L0 = self.layers[0]
         # every key is a cache slot: the "new" K/V views are never read
-        attn = PackedAttention(q, L0["k"].transpose(0, 1), table, k_cache=L0["k"], s_cache=self.capacity, out=o,
-                               v_new=L0["v"].transpose(0, 1), v_cache=L0["v"], max_splits=self.max_splits)
+        attn = PackedAttention._host_planned(q, L0["k"].transpose(0, 1), table, L0["k"], self.capacity, o, L0["v"].transpose(0, 1),
+                                             L0["v"], self.max_splits)
+        # the pass's tables and plan in one asynchronous copy (the host runs
+        # ahead of the GPU; pageable copies made it wait for the last pass)
+        i32 = lambda a: np.asarray(a).astype(np.int32, copy=False)  # noqa: E731
+        ids, pos_d, slots_d, attn.plan.dev = upload_async([i32(tokens), i32(pos), i32(slots), attn.plan.host], self.device)
+        if attn.plan.workspace_bytes:
+            attn.plan.workspace = torch.empty(attn.plan.workspace_bytes, dtype=torch.uint8, device=self.device)
+        gather_rows(self.embed, ids, out=x)
         for i, L in enumerate(self.layers):
             # ln1: the first layer's input is the embedding; later ones come
             # fused with the previous layer's MLP residual add below
@@ -112,7 +117,7 @@ class Qwen3Stack:
         gathered rows only."""
         import torch
         x, h = xh
-        g = torch.as_tensor(np.ascontiguousarray(gather, np.int32), device=self.device)
+        g, = upload_async([np.asarray(gather).astype(np.int32, copy=False)], self.device)
         xg, hg = gather_rows(x, g), gather_rows(h, g)
         y = rms_norm(xg, self.norm, self.w.eps, h=hg, x_out=xg)
         return gather_rows(y, out_dtype=torch.float32)
