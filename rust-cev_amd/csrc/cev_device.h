@@ -47,36 +47,22 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // The bf16 SiLU of a bf16 value, v / (1 + e^-v) with each op rounded to
-// bf16, depends on its 16 bits only.  Kernels that apply it to many values
-// tabulate it in LDS for |v| in [2^-16, 2^7) (23 binades of 128 mantissas
-// per sign), evaluated by the same silu_bf16, so a table hit is
-// bit-identical to evaluating it; values outside take silu_bf16 itself.
-// (The translation units that use it are built without FMA contraction.)
-constexpr uint32_t kSiluLo = (127 - 16) * 128;  // |bits| of 2^-16
-constexpr uint32_t kSiluSpan = 23 * 128;        // entries per sign
-constexpr int kSiluEntries = 2 * (int)kSiluSpan;
-
+// bf16, on the hardware exp2 and reciprocal: 12 instructions, where expf and
+// the f32 division take about 45 (and a table of the values in LDS, which
+// this replaces, cost every workgroup 2.5 us to fill).
+//   e^-v: log2 e in two parts keeps 2^(-v log2 e) within 2 f32 ulps over the
+//   range where it counts; a test compares all 65536 arguments with the
+//   correctly rounded ops.
+//   v / den: den = D 2^p and v = V 2^q with D, V 8-bit integers; a bf16
+//   rounding midpoint is M 2^r with M an odd 9-bit integer, and V = D M has
+//   no solution, so v / den lies at least 2^-17 (relative) from every
+//   midpoint and the 2^-22 error of v * rcp(den) cannot change its rounding.
+//   Both are taken at a quarter (exact), which keeps the reciprocal of a
+//   denominator near 2^128 out of the denormals that the unit flushes.
 __device__ __forceinline__ float silu_bf16(float v) {
-  const float ex = bf16_round(expf(-v));
-  const float den = bf16_round(1.0f + ex);
-  return bf16_round(v / den);
-}
-
-// table slot of a bf16-exact value: negative values after the positive ones;
-// >= kSiluEntries when |v| is outside the table
-__device__ __forceinline__ uint32_t silu_slot(float v) {
-  const uint32_t b = __float_as_uint(v) >> 16;
-  const uint32_t m = (b & 0x7fffu) - kSiluLo;
-  return m < kSiluSpan ? m + (b >> 15) * kSiluSpan : (uint32_t)kSiluEntries;
-}
-
-// Every thread of a workgroup of `threads` fills its share of the table.
-__device__ __forceinline__ void silu_fill(float* tab, int threads) {
-  for (int i = threadIdx.x; i < kSiluEntries; i += threads) {
-    const uint32_t neg = i >= (int)kSiluSpan;
-    const uint32_t bits = (neg << 15) | (kSiluLo + (uint32_t)i - neg * kSiluSpan);
-    tab[i] = silu_bf16(bf16_from_bits((uint16_t)bits));
-  }
+  const float ex = bf16_round(fast_exp2(__builtin_fmaf(v, -1.44269502f, v * -1.92596303e-8f)));
+  const float den4 = bf16_round(__builtin_fmaf(ex, 0.25f, 0.25f));
+  return bf16_round(0.25f * v * __builtin_amdgcn_rcpf(den4));
 }
 
 template <typename Fn, int... I>

@@ -115,29 +115,30 @@ struct GdnArgs {
   float* rec;    // workspace: (B, nv, n_chunks) records
   float* core;   // workspace: (B, T, nv, dv) f32
   int64_t mixed_sb, mixed_st, z_sb, z_st, ab_sb, ab_st, conv_in_sb, s_in_sb, y_sb, y_st;
-  int32_t batch, t, nk, nv, kernel, conv_dim, n_chunks, conv_run;
+  int32_t batch, t, nk, nv, kernel, conv_dim, n_chunks;
+  bool conv_w_vec, conv_in_vec, conv_out_vec;  // 16-byte accesses allowed
   float eps;
 };
 
 // ---------------------------------------------------------------------------
-// conv + SiLU.  Thread = (row, 8 channels, run of conv_run tokens): the 8 x K
-// weights stay in registers and the last K-1 input rows slide through a
-// register window, so every input row is read once as one 16-byte vector.
-// Each product and partial sum is one model-dtype op (decoder.rs:143-150);
-// SiLU is candle's v / (1 + exp(-v)) with each op in the model dtype.  The
-// thread of a row's last run also writes the new conv state: its window then
-// holds the last K-1 columns of [state || x] (qwen35.rs:429).
-// Run length: 16 tokens, or 8 / 4 when that leaves fewer workgroups than
-// CUs (short rows, e.g. 32 rows of 64 tokens).
-constexpr int kConvRunMax = 16;
+// conv + SiLU.  Thread = (row, 8 channels, run of R tokens): the 8 x K
+// weights stay in registers and all R + K - 1 input rows of the run are
+// loaded, 16 bytes each, before the first is used.  Each product and partial
+// sum is one model-dtype op (decoder.rs:143-150); SiLU is candle's
+// v / (1 + exp(-v)) with each op in the model dtype.  The thread of a row's
+// last run also writes the new conv state: the last K-1 columns of
+// [state || x] (qwen35.rs:429).
+// What bounds it: VALU issue in bf16 (the op-by-op rounding, about 34 us over
+// the chip for a 4096-token row, against 26 us for its 134 MB).  Sliding one
+// row ahead through a run of 16 waited for a load per token, and each
+// workgroup first filled a SiLU table in LDS: 54 us, now 43; 32 rows of 64
+// tokens 38 -> 26; f32, 3 x 333 tokens, 26 -> 19; one token 12.3 -> 5.
+// Run length: 8 tokens (46 us at 4 or 5, 45 at 6, on the long row) when that
+// still gives every CU two workgroups, else 4.
+constexpr int kConvThreads = 256;
+constexpr int kConvRunShort = 4;
+constexpr int kConvRunLong = 8;
 constexpr int kConvCus = 256;
-// 16 waves per workgroup share one table; widths 7 and 8 need more than the
-// 128 registers that leaves each lane, so they run 8 waves
-constexpr int conv_threads(int K) { return K <= 6 ? 1024 : 512; }
-
-// Each conv workgroup first tabulates the bf16 SiLU in LDS (silu_fill), and
-// a token whose 8 x 64 values are not all in the table's range takes
-// silu_bf16 itself (wave-uniform branch).
 
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -163,8 +164,7 @@ __device__ __forceinline__ void load8<float>(const float* p, float* v) {
     v[e + 4] = y[e];
   }
 }
-// 8 channels of one input row as loaded (converted to f32 where used, so a
-// row loaded one iteration ahead is not waited for early)
+// 8 channels of one input row as loaded (converted to f32 where used)
 template <typename T>
 struct Raw8;
 template <>
@@ -172,6 +172,7 @@ struct Raw8<__bf16> {
   bf16x8 x;
   __device__ __forceinline__ void load(const __bf16* p) { x = *(const bf16x8*)p; }
   __device__ __forceinline__ float operator[](int e) const { return (float)x[e]; }
+  __device__ __forceinline__ void set(int e, float v) { x[e] = (__bf16)v; }
 };
 template <>
 struct Raw8<float> {
@@ -181,6 +182,12 @@ struct Raw8<float> {
     y = *(const f32x4*)(p + 4);
   }
   __device__ __forceinline__ float operator[](int e) const { return e < 4 ? x[e] : y[e - 4]; }
+  __device__ __forceinline__ void set(int e, float v) {
+    if (e < 4)
+      x[e] = v;
+    else
+      y[e - 4] = v;
+  }
 };
 
 template <typename T>
@@ -198,42 +205,51 @@ __device__ __forceinline__ void store8<float>(float* p, const float* v) {
   *(f32x4*)(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
 }
 
-template <typename T, int K>
-__device__ __forceinline__ void conv_run(const GdnArgs& g, const float* silu_tab, int r, int t0, int c0) {
-  const T* x = (const T*)g.mixed + r * g.mixed_sb;
-  const T* tail = g.conv_in ? (const T*)g.conv_in + r * g.conv_in_sb : nullptr;
-  float w[8][K];
+// 8 x N consecutive model-dtype values as f32: v[e N + u] is column u of
+// channel e.  By 16-byte loads where the address allows it.
+template <typename T, int N>
+__device__ __forceinline__ void load_channels(const T* p, bool vec, float* v) {
+  if (vec) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
+    for (int i = 0; i < N; ++i) load8<T>(p + 8 * i, v + 8 * i);
+  } else {
 #pragma unroll
-    for (int u = 0; u < K; ++u) w[e][u] = to_f(((const T*)g.conv_w)[(int64_t)(c0 + e) * K + u]);
-  // window[j] = input row t - (K-1) + j for the token t being produced
-  float win[K][8];
+    for (int i = 0; i < 8 * N; ++i) v[i] = to_f(p[i]);
+  }
+}
+
+template <typename T, int K, int R>
+__global__ __launch_bounds__(kConvThreads) void gdn_conv_kernel(GdnArgs g) {
+  // block -> (run, block of channels): the divisions are wave-uniform
+  const uint32_t cg = (uint32_t)g.conv_dim / 8, cblocks = (cg + kConvThreads - 1) / kConvThreads;
+  const uint32_t runs = ((uint32_t)g.t + R - 1) / R, rr = blockIdx.x / cblocks;
+  const uint32_t ci = (blockIdx.x - rr * cblocks) * kConvThreads + threadIdx.x;
+  if (ci >= cg) return;
+  const int c0 = (int)ci * 8;
+  const int r = (int)(rr / runs), t0 = (int)(rr - (uint32_t)r * runs) * R;
+  const T* x = (const T*)g.mixed + r * g.mixed_sb + c0;
+  const T* tail = g.conv_in ? (const T*)g.conv_in + r * g.conv_in_sb + (int64_t)c0 * (K - 1) : nullptr;
+  // rows[j] = input row t0 - (K-1) + j; rows past the end repeat the last
+  Raw8<T> rows[R + K - 1];
 #pragma unroll
-  for (int j = 0; j < K - 1; ++j) {
-    const int p = t0 - (K - 1) + j;
-    if (p >= 0) {
-      load8<T>(x + (int64_t)p * g.mixed_st + c0, win[j]);
-    } else {
+  for (int j = 0; j < R + K - 1; ++j) rows[j].load(x + (int64_t)min(max(t0 - (K - 1) + j, 0), g.t - 1) * g.mixed_st);
+  float w[8 * K];
+  load_channels<T, K>((const T*)g.conv_w + (int64_t)c0 * K, g.conv_w_vec, w);
+  if (t0 < K - 1) {  // the rows before the first come from the state: row t0 - (K-1) + j is its column t0 + j
+    static_assert(2 * R >= K - 1, "at most the first two runs reach into the state");
+    float tv[8 * (K - 1)] = {};
+    if (tail) load_channels<T, K - 1>(tail, g.conv_in_vec, tv);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) win[j][e] = tail ? to_f(tail[(int64_t)(c0 + e) * (K - 1) + (K - 1 + p)]) : 0.0f;
-    }
+    for (int j = 0; j < K - 1; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (t0 == 0) rows[j].set(e, tv[e * (K - 1) + j]);
+        if (R + j < K - 1 && t0 == R) rows[j].set(e, tv[e * (K - 1) + min(R + j, K - 2)]);
+      }
   }
   T* out = (T*)g.conved + ((int64_t)r * g.t + t0) * g.conv_dim + c0;
-  const int n = min(g.conv_run, g.t - t0);
-  // the next row loads while this one is computed (the last load repeats
-  // the last row, so it stays unconditional and in bounds)
-  Raw8<T> next;
-  const T* xp = x + (int64_t)t0 * g.mixed_st + c0;
-  next.load(xp);
-  // s_waitcnt vmcnt(0): with nothing pending at the loop entry, the wait at
-  // the loop head covers only the prefetch, not the previous row's store
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  for (int i = 0; i < n; ++i) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) win[K - 1][e] = next[e];
-    xp += i + 1 < n ? g.mixed_st : 0;
-    next.load(xp);
+  for (int i = 0; i < R; ++i) {
     float y[8];
     if constexpr (sizeof(T) == 2) {
       // products and partial sums, each rounded to bf16, two channels per
@@ -243,84 +259,73 @@ __device__ __forceinline__ void conv_run(const GdnArgs& g, const float* silu_tab
       for (int u = 0; u < K; ++u)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x2v term = bf16_round2(f32x2v{win[u][2 * q] * w[2 * q][u], win[u][2 * q + 1] * w[2 * q + 1][u]});
+          const f32x2v term = bf16_round2(f32x2v{rows[i + u][2 * q] * w[2 * q * K + u], rows[i + u][2 * q + 1] * w[(2 * q + 1) * K + u]});
           acc[q] = u == 0 ? term : bf16_round2(acc[q] + term);
         }
-      uint32_t slot[8];
-      bool hit = true;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        slot[e] = silu_slot(acc[e / 2][e % 2]);
-        hit = hit && slot[e] < (uint32_t)kSiluEntries;
-      }
-      if (__all(hit)) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = silu_tab[slot[e]];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] = silu_bf16(acc[e / 2][e % 2]);
-      }
+      for (int e = 0; e < 8; ++e) y[e] = silu_bf16(acc[e / 2][e % 2]);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float acc = 0.0f;
 #pragma unroll
-        for (int u = 0; u < K; ++u) acc = u == 0 ? win[u][e] * w[e][u] : acc + win[u][e] * w[e][u];
+        for (int u = 0; u < K; ++u) acc = u == 0 ? rows[i + u][e] * w[e * K + u] : acc + rows[i + u][e] * w[e * K + u];
         y[e] = acc / (1.0f + expf(-acc));
       }
     }
-    store8<T>(out + (int64_t)i * g.conv_dim, y);
-#pragma unroll
-    for (int j = 0; j < K - 1; ++j)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) win[j][e] = win[j + 1][e];
+    if (t0 + i < g.t) store8<T>(out + (int64_t)i * g.conv_dim, y);
   }
-  if (t0 + n == g.t) {
-    // new conv state (conv_dim, K-1) of this row: the window's last K-1 columns
-    T* st = (T*)g.conv_out + ((int64_t)r * g.conv_dim + c0) * (K - 1);
+  if (t0 + R >= g.t) {
+    // new conv state (conv_dim, K-1) of this row, read again by its place
+    float st[8 * (K - 1)], tv[8 * (K - 1)] = {};
+    if (g.t < K - 1 && tail) load_channels<T, K - 1>(tail, g.conv_in_vec, tv);
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
+    for (int j = 0; j < K - 1; ++j) {
+      const int p = g.t - (K - 1) + j;
+      Raw8<T> row;
+      row.load(x + (int64_t)max(p, 0) * g.mixed_st);
 #pragma unroll
-      for (int j = 0; j < K - 1; ++j) st[e * (K - 1) + j] = from_f<T>(win[j][e]);
+      for (int e = 0; e < 8; ++e) {
+        float v = row[e];
+#pragma unroll
+        for (int u = 0; u < K - 1; ++u) v = p + (K - 1) == u ? tv[e * (K - 1) + u] : v;  // p < 0: column K-1+p of the old state
+        st[e * (K - 1) + j] = v;
+      }
+    }
+    T* so = (T*)g.conv_out + ((int64_t)r * g.conv_dim + c0) * (K - 1);
+    if (g.conv_out_vec) {
+#pragma unroll
+      for (int i = 0; i < K - 1; ++i) store8<T>(so + 8 * i, st + 8 * i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8 * (K - 1); ++i) so[i] = from_f<T>(st[i]);
+    }
   }
 }
 
-// One kernel per conv width, so each gets its own register allocation (the
-// window and weights take 16 K registers).
+// One kernel per conv width and run length, so each gets its own register
+// allocation.
 template <typename T, int K>
-__global__ __launch_bounds__(conv_threads(K)) void gdn_conv_kernel(GdnArgs g) {
-  constexpr int kConvThreads = conv_threads(K);
-  __shared__ float silu_tab[sizeof(T) == 2 ? kSiluEntries : 1];
-  if constexpr (sizeof(T) == 2) {
-    silu_fill(silu_tab, kConvThreads);
-    __syncthreads();
-  }
-  const int64_t cg = g.conv_dim / 8;
-  const int64_t runs = (g.t + g.conv_run - 1) / g.conv_run;
-  const int64_t idx = (int64_t)blockIdx.x * kConvThreads + threadIdx.x;
-  if (idx >= (int64_t)g.batch * runs * cg) return;
-  const int c0 = (int)(idx % cg) * 8;
-  const int64_t rr = idx / cg;
-  const int t0 = (int)(rr % runs) * g.conv_run, r = (int)(rr / runs);
-  conv_run<T, K>(g, silu_tab, r, t0, c0);
-}
-
-template <typename T, int K>
-void launch_conv_k(const GdnArgs& g, int64_t items, hipStream_t s) {
-  constexpr int n = conv_threads(K);
-  hipLaunchKernelGGL((gdn_conv_kernel<T, K>), dim3((unsigned)((items + n - 1) / n)), dim3(n), 0, s, g);
+void launch_conv_k(const GdnArgs& g, bool long_runs, hipStream_t s) {
+  const int R = long_runs ? kConvRunLong : kConvRunShort;
+  const int64_t cblocks = (g.conv_dim / 8 + kConvThreads - 1) / kConvThreads;
+  const dim3 grid((unsigned)((int64_t)g.batch * ((g.t + R - 1) / R) * cblocks)), block(kConvThreads);
+  if (long_runs)
+    hipLaunchKernelGGL((gdn_conv_kernel<T, K, kConvRunLong>), grid, block, 0, s, g);
+  else
+    hipLaunchKernelGGL((gdn_conv_kernel<T, K, kConvRunShort>), grid, block, 0, s, g);
 }
 
 template <typename T>
-void launch_conv(const GdnArgs& g, int64_t items, hipStream_t s) {
+void launch_conv(const GdnArgs& g, bool long_runs, hipStream_t s) {
   switch (g.kernel) {
-    case 2: launch_conv_k<T, 2>(g, items, s); break;
-    case 3: launch_conv_k<T, 3>(g, items, s); break;
-    case 4: launch_conv_k<T, 4>(g, items, s); break;
-    case 5: launch_conv_k<T, 5>(g, items, s); break;
-    case 6: launch_conv_k<T, 6>(g, items, s); break;
-    case 7: launch_conv_k<T, 7>(g, items, s); break;
-    default: launch_conv_k<T, 8>(g, items, s); break;
+    case 2: launch_conv_k<T, 2>(g, long_runs, s); break;
+    case 3: launch_conv_k<T, 3>(g, long_runs, s); break;
+    case 4: launch_conv_k<T, 4>(g, long_runs, s); break;
+    case 5: launch_conv_k<T, 5>(g, long_runs, s); break;
+    case 6: launch_conv_k<T, 6>(g, long_runs, s); break;
+    case 7: launch_conv_k<T, 7>(g, long_runs, s); break;
+    default: launch_conv_k<T, 8>(g, long_runs, s); break;
   }
 }
 
@@ -1376,22 +1381,23 @@ extern "C" int32_t cev_gdn_forward(const cev_gdn_desc* d, const void* mixed, con
   g.n_chunks = (d->t + kC - 1) / kC;
   g.eps = d->eps;
   hipStream_t s = (hipStream_t)stream;
-  const int conv_wg = conv_threads(g.kernel);
-  auto conv_items_of = [&](int run) { return (int64_t)g.batch * ((g.t + run - 1) / run) * (g.conv_dim / 8); };
-  g.conv_run = kConvRunMax;
-  while (g.conv_run > 4 && conv_items_of(g.conv_run) < (int64_t)kConvCus * conv_wg) g.conv_run /= 2;
-  const int64_t conv_items = conv_items_of(g.conv_run);
+  auto aligned = [](const void* p, int64_t stride_bytes) { return (((uintptr_t)p | (uintptr_t)stride_bytes) & 15) == 0; };
+  g.conv_w_vec = aligned(conv_w, 0);
+  g.conv_in_vec = aligned(conv_in, g.conv_in_sb * (int64_t)esz);
+  g.conv_out_vec = aligned(conv_out, 0);  // a channel's K - 1 columns, 8 channels: 16 (K - 1) bytes or more
+  const int64_t conv_items = (int64_t)g.batch * ((g.t + kConvRunLong - 1) / kConvRunLong) * (g.conv_dim / 8);
+  const bool long_runs = conv_items >= 2 * (int64_t)kConvCus * kConvThreads;
   const int64_t recs = (int64_t)g.batch * g.nv * g.n_chunks;
   // scan grid: (bf16, many chunks) groups of value heads per key head, rounded up to the 8 XCDs, x group size x slices
   const int64_t grp = d->dtype == CEV_BF16 && g.n_chunks > 1 ? g.nv / g.nk : 1;
   const int64_t slices = ((int64_t)g.batch * g.nv / grp + kXcds - 1) / kXcds * kXcds * grp * (kD / kW);
   const int64_t norm_items = (int64_t)g.batch * g.t * g.nv;
-  if (recs > INT32_MAX || (conv_items + 511) / 512 > INT32_MAX) return cev_fail(CEV_ERR_UNSUPPORTED, "GDN grid too large");
+  if (recs > INT32_MAX || (int64_t)g.batch * ((g.t + kConvRunShort - 1) / kConvRunShort) * ((g.conv_dim / 8 + kConvThreads - 1) / kConvThreads) > INT32_MAX) return cev_fail(CEV_ERR_UNSUPPORTED, "GDN grid too large");
   if (d->dtype == CEV_BF16) {
-    launch_conv<__bf16>(g, conv_items, s);
+    launch_conv<__bf16>(g, long_runs, s);
     hipLaunchKernelGGL(gdn_prep_kernel<__bf16>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
   } else {
-    launch_conv<float>(g, conv_items, s);
+    launch_conv<float>(g, long_runs, s);
     hipLaunchKernelGGL(gdn_prep_kernel<float>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
   }
   const bool bf = d->dtype == CEV_BF16;

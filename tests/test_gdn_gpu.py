@@ -347,3 +347,52 @@ def test_gdn_graph_replay_matches_eager(gpu):
         torch.cuda.synchronize()
         for got, ref in zip((y, co, so), want):
             assert np.array_equal(to_np(got), ref), f"replay {i}"
+
+
+def test_silu_of_every_bf16_value(gpu):
+    """The bf16 SiLU on the hardware exp2 and reciprocal equals the correctly
+    rounded op sequence (e^-v, 1 + e, v / den, each to bf16) for all 65536
+    arguments; seen through swiglu with up = 1."""
+    import torch
+    v = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(64, 1024)
+    got = cev_hip.swiglu(v.to(gpu), torch.ones_like(v, device=gpu)).cpu().double()
+
+    def to_bf16(x):  # one rounding from f64: the f32 in between is moved off a false tie
+        x = x.numpy()
+        with np.errstate(over="ignore"):
+            f = x.astype(np.float32)
+        b = f.view(np.uint32).copy()
+        tie, a = (b & 0xFFFF) == 0x8000, np.abs(f.astype(np.float64))
+        b[tie & (np.abs(x) > a)] += 1
+        b[tie & (np.abs(x) < a)] -= 1
+        return torch.from_numpy(b.view(np.float32)).bfloat16().double()
+
+    d = v.double()
+    want = to_bf16(d / to_bf16(1.0 + to_bf16(torch.exp(-d))))
+    same = (got == want) | (got.isnan() & want.isnan())
+    assert same.all(), d[~same]
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("t", [1, 2, 3, 4, 7, 9, 300])
+def test_conv_on_unaligned_views(gpu, bf16, t):
+    """Conv weights and state at addresses that no 16-byte load may touch, and
+    runs that start, end and lie inside the state's columns, give what aligned
+    copies of them give."""
+    import torch
+    B, nk, nv, K = 2, 2, 4, 4
+    dt = torch.bfloat16 if bf16 else torch.float32
+    dim = (2 * nk + nv) * 128
+    g = torch.Generator().manual_seed(t)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dt).to(gpu)  # noqa: E731
+    mixed, z, b, a = rnd(B, t, dim), rnd(B, t, nv * 128), rnd(B, t, nv), rnd(B, t, nv)
+    w, state = rnd(dim * K + 1), rnd(B * dim * (K - 1) + 1)
+    f = lambda n, v: torch.full((n,), v, device=gpu)  # noqa: E731
+    layer = cev_hip.GatedDeltaNet(B, t, nk, nv, dtype=dt, device=gpu)
+    run = lambda w_, s_: layer(mixed, z, b, a, w_, f(nv, -1.0), f(nv, 0.0), f(128, 1.0), conv_in=s_)  # noqa: E731
+    w1, s1 = w[1:].view(dim, K), state[1:].view(B, dim, K - 1)
+    got, want = run(w1, s1), run(w1.clone(), s1.clone())
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    seq = torch.cat([s1, mixed.transpose(1, 2)], 2)
+    assert torch.equal(got[1], seq[:, :, t:])
