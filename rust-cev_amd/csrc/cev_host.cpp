@@ -264,7 +264,7 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
   const int g = d->n_q_heads / d->n_kv_heads;
   const bool bf = d->dtype == CEV_BF16, wide = d->head_dim == 256;
   const int32_t sub_rows = 32 / g;
-  int64_t rows = 0, n_subs = 0;
+  int64_t rows = 0, n_subs = 0, all_chunks = 0;
   int32_t max_rows = 0, max_chunks = 0;
   for (int32_t ti = 0; ti < p.n_tiles; ++ti) {
     const int32_t* t = &p.tiles[(size_t)ti * 8];
@@ -272,6 +272,7 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
     n_subs += (t[1] + sub_rows - 1) / sub_rows;
     max_rows = std::max(max_rows, t[1]);
     max_chunks = std::max(max_chunks, t[4]);
+    all_chunks += t[4];
   }
   // max_splits = 1 asks for one walk over every row's keys in stream order;
   // beyond 16 workgroups a CU the 256-slot kernels fill the chip
@@ -281,8 +282,10 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
   };
   // 256-slot kernels
   const double f = (double)max_rows / p.tile_rows;
-  const int64_t wgs = (int64_t)p.n_tiles * d->n_kv_heads * p.n_splits;
-  const double steps = (double)((wgs + kSplitTargetWorkgroups - 1) / kSplitTargetWorkgroups) * ((max_chunks + p.n_splits - 1) / p.n_splits);
+  // (the longer of the longest part and an even share of all chunks: a tile
+  // that meets two blocks' keys must not stand for all of them)
+  const double steps = std::max((double)((max_chunks + p.n_splits - 1) / p.n_splits),
+                                (double)(all_chunks * d->n_kv_heads) / kSplitTargetWorkgroups);
   double whole = merge_us(p.n_splits);
   if (!bf)
     whole += 8.0 + steps * (f > 0.5 ? 8.2 : 4.2);
