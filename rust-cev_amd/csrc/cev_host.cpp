@@ -318,19 +318,23 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
         sum_rounds += rounds;
       }
     }
-    const double w = (double)(n_subs * d->n_kv_heads * parts), cus = kSplitTargetWorkgroups;
+    // launched workgroups, the empty ones of short tiles too: they shift the
+    // others so that some CUs get one more (481 rows in 320 workgroups, 62
+    // of them empty, took two CU rounds: 42 us against 35 in 256-slot form)
+    const int32_t subs_per_tile = (max_rows + sub_rows - 1) / sub_rows;
+    const double cu_rounds = std::ceil((double)((int64_t)p.n_tiles * subs_per_tile * d->n_kv_heads * parts) / kSplitTargetWorkgroups);
     const double r = (double)max_rounds, avg = (double)sum_rounds / (double)n_subs;
     double us = merge_us(parts);
     if (!bf)
-      us += 6.0 + 5.2 * std::max(r, std::ceil(w / cus) * avg);
+      us += 6.0 + 5.2 * std::max(r, cu_rounds * avg);
     else if (wide)
-      us += 3.0 + std::max(10.0 + 2.0 * r, std::ceil(w / cus) * (10.0 + 2.0 * avg));
+      us += 3.0 + std::max(10.0 + 2.0 * r, cu_rounds * (10.0 + 2.0 * avg));
     else
-      us += 6.0 + std::max(1.2 * r, w / cus * (1.25 * avg + 1.6));
+      us += 6.0 + std::max(1.2 * r, cu_rounds * (1.25 * avg + 1.6));
     if (us < best) {
       best = us;
       p.fan_parts = (int32_t)parts;
-      p.fan_subs = (max_rows + sub_rows - 1) / sub_rows;
+      p.fan_subs = subs_per_tile;
     }
   }
 }
