@@ -18,6 +18,7 @@
 // All chunk-rule products run on v_mfma_f32_16x16x4_f32 (full f32 like the
 // reference).  Lane layout (16x16x4): A lane l holds A[l%16][l/16], B lane l
 // holds B[l/16][l%16], D lane l register r holds D[4(l/16)+r][l%16].
+#include <cmath>
 #include <cstring>
 
 #include <type_traits>
@@ -50,13 +51,10 @@ constexpr int kSC = 68;    // LDS row stride of 64-wide f32 tiles
 // The scan rebuilds Qd = (q * Qf0) * Qf1 and Kd = (k * 1/|k|) * e^(last - cum)
 // with prep's own two roundings, so both layouts give the same bits; the bf16
 // record is 113 KB instead of 144 KB.  Qb and Kb depend on the key head only:
-// for the many-chunk scan the first value head of each key head's group writes
-// them, and the scans of the group's other value heads read them from that
-// head's record.
-// In's six tiles above the diagonal are zero.  The scan skips their MFMAs,
-// and the many-chunk scan never loads them either, so prep stores them only
-// for the one-chunk scan, which loads every tile at a fixed offset (it is
-// held to 128 registers, and the clamped addresses cost it spills).
+// the first value head of each key head's group writes them, and the scans of
+// the group's other value heads read them from that head's record.
+// In's six tiles above the diagonal are zero: prep never stores them and the
+// scan neither loads nor multiplies them.
 template <bool BF>
 struct RecLayout;
 template <>
@@ -116,7 +114,7 @@ struct GdnArgs {
   float* core;   // workspace: (B, T, nv, dv) f32
   int64_t mixed_sb, mixed_st, z_sb, z_st, ab_sb, ab_st, conv_in_sb, s_in_sb, y_sb, y_st;
   int32_t batch, t, nk, nv, kernel, conv_dim, n_chunks;
-  bool conv_w_vec, conv_in_vec, conv_out_vec;  // 16-byte accesses allowed
+  bool conv_w_vec, conv_in_vec, conv_out_vec, norm_vec;  // 16-byte accesses allowed
   float eps;
 };
 
@@ -517,11 +515,8 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_prep_kernel(GdnArgs g) {
   const int hr = blockIdx.x / g.n_chunks;
   const int h = hr % g.nv, r = hr / g.nv;
   const int kh = h / (g.nv / g.nk);  // value head h reads key head h / (nv/nk) (qwen35.rs:436-442)
-  // bf16 records for the many-chunk scan: only the group's first value head
-  // stores the raw q / k rows (the one-chunk scan reads its own record's)
-  const bool qk_rows = !BF || g.n_chunks == 1 || h % (g.nv / g.nk) == 0;
-  // intra's zero tiles: read only by the one-chunk scan
-  const bool zero_tiles = g.n_chunks == 1;
+  // bf16 records: only the group's first value head stores the raw q / k rows
+  const bool qk_rows = !BF || h % (g.nv / g.nk) == 0;
   const int key_dim = g.nk * kD;
   const int t0 = c * kC;
   const T* cv = (const T*)g.conved + (int64_t)r * g.t * g.conv_dim;
@@ -682,8 +677,7 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_prep_kernel(GdnArgs g) {
   };
   // Records the inversion's idle waves write: q e^cum (Qd) and k e^(last -
   // cum) (Kd) in their fragment orders (bf16 models: the raw rows, from the
-  // group's first value head only, and every head's factors), and for the
-  // one-chunk scan intra's six zero tiles.
+  // group's first value head only, and every head's factors).
   constexpr int kQdStores = BF ? kC * kD / 8 : kC * kD / 4;  // 16-byte stores per record part
   auto qd_records = [&](int p0, int step) {
     for (int p = p0; p < kQdStores; p += step) {
@@ -742,14 +736,6 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_prep_kernel(GdnArgs g) {
     }
   };
 
-  auto zero_intra = [&](int p0, int step) {
-    for (int p = p0; p < 6 * 64; p += step) {
-      const int q = p >> 6;  // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
-      const int ti = q < 3 ? 0 : (q < 5 ? 1 : 2), tj = q < 3 ? q + 1 : (q < 5 ? q - 1 : 3);
-      *(f32x4*)(rec + R::In + 4 * ((ti * 4 + tj) * 64 + (p & 63))) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-  };
-
   // kc operands of this wave's column tile: (k beta) e^cum
   // (qwen35.rs:309-312, :336-340), in the same k order as vreg
   auto operands = [&]() {
@@ -800,7 +786,6 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_prep_kernel(GdnArgs g) {
     for (int e = 0; e < 4; ++e) L.Tm[(16 * ti2 + 4 * fq + e) * kSC + 16 * tj2 + fm] = bc[e];
   } else {
     if (qk_rows) kd_records(tid - 256, kQdStores / 2, 256);
-    if (zero_tiles) zero_intra(tid - 256, 256);
     factor_records(tid - 256);
   }
   __syncthreads();
@@ -868,7 +853,7 @@ __global__ __launch_bounds__(kPrepThreads) void gdn_prep_kernel(GdnArgs g) {
 //     chunk's output at the start of the next chunk.
 // The A operands come straight from the fragment-ordered record (L2), the
 // B operands (S, v_new) from LDS.  blockIdx -> (item, slice) keeps the 8
-// slices of one head, and in the bf16 many-chunk scan the value heads of one
+// slices of one head, and in the bf16 scan the value heads of one
 // key head, on one XCD (workgroups go round-robin over the 8 XCDs), so each
 // head's records, and the raw q / k rows the group shares, are fetched into
 // one L2 only.
@@ -893,29 +878,26 @@ struct ScanOps<true> {
   float decay;
 };
 
-template <bool kPrefetch, bool BF>
-__device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
+template <bool BF>
+__global__ __launch_bounds__(kScanThreads) void gdn_scan_kernel(GdnArgs g) {
   using R = RecLayout<BF>;
   using Ops = ScanOps<BF>;
-  // 16-column tiles.  The prefetching loop stores row r at row
-  // r ^ ((r >> 2) & 3) of a 16-float stride: the B-operand reads (rows
-  // 4i .. 4i+3 across a wave) and the accumulator writes (rows 4fq + e) then
-  // both touch 64 distinct banks.  The one-chunk kernel keeps a 20-float
-  // stride (2-way conflicts on the reads): the swizzle's extra address
-  // registers would not fit its 128.
-  constexpr int kRow = kPrefetch ? 16 : 20;
+  // 16-column tiles that store row r at row r ^ ((r >> 2) & 3) of a 16-float
+  // stride: the B-operand reads (rows 4i .. 4i+3 across a wave) and the
+  // accumulator writes (rows 4fq + e) then both touch 64 distinct banks.
+  constexpr int kRow = 16;
   __shared__ float S[kD * kRow];     // state slice (dk x 16), updated in place
   __shared__ float Vn0[kC * kRow];   // new_values - k_cumdecay . S, first half of dk
   __shared__ float Vn1[kC * kRow];   // k_cumdecay . S, second half of dk
   __shared__ float Opart[kC * kRow]; // (q e^cum) . S, second half of dk
   __shared__ float KF[BF ? 2 * kC : 1];  // bf16: the chunk's Kf array
-  auto sx = [](int row, int col) { return kPrefetch ? (row ^ ((row >> 2) & 3)) * 16 + col : row * 20 + col; };
+  auto sx = [](int row, int col) { return (row ^ ((row >> 2) & 3)) * 16 + col; };
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int rt = wave & 3, kh = wave >> 2;
   constexpr int nslice = kD / kW;
-  // value heads that share one key head's q / k rows (bf16 records, many-chunk scan)
-  const int grp = BF && kPrefetch ? g.nv / g.nk : 1;
+  // value heads that share one key head's q / k rows (bf16 records)
+  const int grp = BF ? g.nv / g.nk : 1;
   // workgroup b runs on XCD b % 8; the groups G = item / grp with G % 8 ==
   // that XCD take its workgroups, slice fastest, then group member m
   const int b = blockIdx.x, y = b / kXcds;
@@ -924,10 +906,8 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
   if (item >= g.batch * g.nv) return;
   const int h = item % g.nv, r = item / g.nv;
   // float offset from this head's record to its group's first head's, which
-  // holds the raw q / k rows for the many-chunk scan.  The one-chunk scan,
-  // held to 128 registers, reads its own record's copy: the second base
-  // address took it from 124 registers to its cap of 128.
-  const int64_t lead_off = kPrefetch ? -(int64_t)m * g.n_chunks * R::Floats : 0;
+  // holds the raw q / k rows
+  const int64_t lead_off = -(int64_t)m * g.n_chunks * R::Floats;
   const int col0 = sl * kW;
   const int fm = lane & 15, fq = lane >> 4;
 
@@ -938,7 +918,7 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
   const int qd_off = BF ? R::Qd + 8 * ((rt * 2 + kh) * 64 + lane) : R::Qd + 4 * (rt * 8 * 64 + 4 * kh * 64 + lane);
   const int kd_off = BF ? R::Kd + 8 * (wave * 64 + lane) : R::Kd + 4 * (wave * 4 * 64 + lane);
   // intra blocks kh and kh + 2 of row tile rt.  Blocks above the diagonal
-  // are zero and their MFMAs are skipped; the many-chunk loop reads the
+  // are zero and their MFMAs are skipped; the loop reads the
   // diagonal block in their place (a line the wave pair reads anyway), so
   // prep need not store them
   const int in_off = R::In + 4 * (rt * 4 * 64 + kh * 64 + lane);
@@ -958,9 +938,9 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
   auto fetch_a = [&](const float* rec, Ops& o, int j) {
     o.kc[j] = ld4(rec + kc_off + 256 * j);
     if (j == 3) {
-      // kh = 1 waves do not use new_values; the prefetching loop loads it
-      // anyway (loads under a branch defeat the compiler's wait tracking there)
-      o.nvv = (kPrefetch || kh == 0) ? ld4(rec + nv_off) : f32x4{};
+      // kh = 1 waves do not use new_values but load it anyway (loads under a
+      // branch defeat the compiler's wait tracking here)
+      o.nvv = ld4(rec + nv_off);
       o.decay = rec[R::Decay];
       if constexpr (BF) o.kf = ld2(rec + kf_off);
     }
@@ -976,7 +956,7 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
       o.qd[j] = ld4(rec + qd_off + 256 * j);
       o.kd[j] = ld4(rec + kd_off + 256 * j);
     }
-    if (j < 2) o.in[j] = kPrefetch ? ld4(rec + in_off + (j == 0 ? in_d0 : in_d1)) : ld4(rec + in_off + 512 * j);
+    if (j < 2) o.in[j] = ld4(rec + in_off + (j == 0 ? in_d0 : in_d1));
   };
   auto fetch = [&](const float* rec, Ops& o) {
 #pragma unroll
@@ -1001,7 +981,7 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
       }
     }
   };
-  // One chunk.  With kPrefetch the next chunk's operands (nrec) load into
+  // One chunk.  The next chunk's operands (nrec) load into
   // nxt one phase ahead of their use, a few loads after each group of four
   // MFMAs: phase A loads the next phase A's k_cumdecay, new_values and decay,
   // phase B the next phase B's operands.  Each wave issues 15 16-byte loads
@@ -1019,16 +999,14 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
     // bf16: q e^cum and k e^(last - cum) are rebuilt here, one k-step group
     // per MFMA group, so the VALU work runs beside the chain and phase B's
     // MFMAs read finished operands; the k factors of this lane's tokens
-    // 4m + fq come from the chunk's Kf array in LDS
-    // (read ahead of the MFMAs in the prefetching loop; the one-chunk
-    // kernel, held to 128 registers, reads each group's just before use)
+    // 4m + fq come from the chunk's Kf array in LDS (read ahead of the MFMAs)
     f32x4 kf4[BF ? 4 : 1], ek4[BF ? 4 : 1];
     float qdf[BF ? 16 : 1], kdf[BF ? 16 : 1];
     auto k_factors = [&](int j) {
       kf4[j] = *(const f32x4*)(KF + 16 * fq + 4 * j);
       ek4[j] = *(const f32x4*)(KF + kC + 16 * fq + 4 * j);
     };
-    if constexpr (BF && kPrefetch) {
+    if constexpr (BF) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) k_factors(j);
     }
@@ -1039,18 +1017,15 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc = mma16(cur.kc[j][e], sb[4 * j + e], acc);
       if constexpr (BF) {
-        if constexpr (!kPrefetch) k_factors(j);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           qdf[4 * j + e] = ((float)cur.qb[j >> 1][(j & 1) * 4 + e] * cur.qf[0]) * cur.qf[1];
           kdf[4 * j + e] = ((float)cur.kb[j >> 1][(j & 1) * 4 + e] * kf4[j][e]) * ek4[j][e];
         }
       }
-      if (kPrefetch) {
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_a(nrec, nxt, j);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_a(nrec, nxt, j);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1082,11 +1057,9 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
         su = mma16(kd, vb[4 * j + e], su);
         ob = mma16(qd, sb[4 * j + e], ob);
       }
-      if (kPrefetch) {
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_b(nrec, nxt, j);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      __builtin_amdgcn_sched_barrier(0);
+      fetch_b(nrec, nxt, j);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // intra . v_new: intra is lower triangular (K stops at the diagonal
     // block); blocks j = kh, kh + 2 go to this wave so the two halves share it
@@ -1118,9 +1091,8 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
       S[sx(r0, fm)] = S[sx(r0, fm)] * cur.decay + su[e];
     }
     // the next chunk's Kf array, read in its phase A; every wave writes the
-    // same values (keeps the load unconditional).  Only the prefetching loop
-    // has a next chunk: the one-chunk kernel runs a single chunk.
-    if constexpr (BF && kPrefetch) *(f32x2v*)(KF + 2 * lane) = nxt.kf;
+    // same values (keeps the load unconditional)
+    if constexpr (BF) *(f32x2v*)(KF + 2 * lane) = nxt.kf;
     __syncthreads();
   };
   Ops ops_a, ops_b;
@@ -1131,42 +1103,22 @@ __device__ __forceinline__ void gdn_scan(const GdnArgs& g) {
   }
   if constexpr (BF) *(f32x2v*)(KF + 2 * lane) = ops_a.kf;  // chunk 0's
   __syncthreads();
-  if constexpr (kPrefetch) {
-    // Two chunks per iteration so the operand sets alternate without a copy
-    // (a copy would wait for every prefetch to land).  The prefetch address
-    // is clamped to the last chunk: the loads stay unconditional, because a
-    // branch around them made the compiler's wait tracking give up.
-    const int last = g.n_chunks - 1;
-    int c = 0;
-    for (; c + 1 < g.n_chunks; c += 2) {
-      chunk(c, ops_a, ops_b, rec_at(c + 1));
-      chunk(c + 1, ops_b, ops_a, rec_at(min(c + 2, last)));
-    }
-    if (c < g.n_chunks) chunk(c, ops_a, ops_b, rec_at(last));
-  } else {
-    for (int c = 0; c < g.n_chunks; ++c) {
-      if (c > 0) fetch(rec_at(c), ops_a);
-      chunk(c, ops_a, ops_a, nullptr);
-    }
+  // Two chunks per iteration so the operand sets alternate without a copy
+  // (a copy would wait for every prefetch to land).  The prefetch address
+  // is clamped to the last chunk: the loads stay unconditional, because a
+  // branch around them made the compiler's wait tracking give up.
+  const int last = g.n_chunks - 1;
+  int c = 0;
+  for (; c + 1 < g.n_chunks; c += 2) {
+    chunk(c, ops_a, ops_b, rec_at(c + 1));
+    chunk(c + 1, ops_b, ops_a, rec_at(min(c + 2, last)));
   }
+  if (c < g.n_chunks) chunk(c, ops_a, ops_b, rec_at(last));
   store_out(g.n_chunks - 1);
   for (int p = tid; p < kD * kW; p += kScanThreads) {
     const int i = p / kW, j = p % kW;
     g.s_out[((int64_t)r * g.nv + h) * kD * kD + (int64_t)i * kD + col0 + j] = S[sx(i, j)];
   }
-}
-
-// Many chunks: the prefetching loop (up to 256 VGPRs, one workgroup per CU).
-template <bool BF>
-__global__ __launch_bounds__(kScanThreads) void gdn_scan_kernel(GdnArgs g) {
-  gdn_scan<true, BF>(g);
-}
-// One chunk per (row, head): no loop to prefetch across, so the registers
-// are held to 128 and two workgroups share a CU, one loading while the
-// other computes.
-template <bool BF>
-__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(4))) void gdn_scan_one_chunk_kernel(GdnArgs g) {
-  gdn_scan<false, BF>(g);
 }
 
 // ---------------------------------------------------------------------------
@@ -1252,6 +1204,446 @@ __global__ __launch_bounds__(256) void gdn_norm_vec_kernel(GdnArgs g) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// prep, scan and norm in one kernel: one workgroup (8 waves) per (row, value
+// head) walks the row's chunks with the whole 128 x 128 state in registers.
+// What it saves: the chunk records (113-147 KB each, written once and read by
+// eight scan workgroups), the f32 core and two launches; what bounds it: one
+// chunk's chain of dependent steps, 14-15 us in bf16 (loads 3, tiles and the
+// diagonal inverses 5, state products 3, the solve and out 4, update and norm
+// 3), with one workgroup a CU.  prep + scan + norm -> this, with the conv:
+// 32 x 64 bf16 rows 190 -> 106 us, 28 x 14 145 -> 59, 5 x 2 45 -> 19,
+// 8 x 383 268 -> 120; f32 9 x 78 140 -> 97.  use_fused draws the line.
+//
+// Wave w owns state columns 16w .. 16w+15 in the f32 accumulator layout
+// (lane (fm, fq): S[16 ti + 4 fq + e][16 w + fm]), which is also the B
+// operand of a 32-deep bf16 MFMA step if its K slots 8 fq + j stand for the
+// rows 32 s + 16 (j / 4) + 4 fq + j % 4; so nothing of the state moves
+// between the products and the update.  Per chunk, as the reference but with
+// the correction taken before the inverse (inv (v beta) - k_cumdecay S =
+// inv (beta (v - e^cum k S))):
+//   ks = k S, qs = q S;   v_new = inv (beta (v - e^cum ks));
+//   out = e^cum qs + intra v_new;   S = S e^last + (k e^(last - cum))^T v_new.
+// The products with q and k run on v_mfma_f32_16x16x32_bf16, eight times the
+// f32 unit's rate, without losing bits: an f32 factor is split into three
+// bf16 parts whose sum is exact, bf16 models' q and k are one part (three
+// products, each exact in f32), f32 models' are three (six products; the
+// dropped ones are below 2^-26).  inv and intra stay on the f32 unit.
+// Chunks of fewer than 64 tokens skip the row tiles past the end.
+template <typename T>
+struct __attribute__((aligned(16))) FusedLds {
+  static constexpr int NA = sizeof(T) == 2 ? 1 : 3;  // bf16 parts of q and k
+  float betas[kC], cums[kC], ecum[kC], ekd[kC], qf[kC], kf[kC];
+  float decay[4];
+  __bf16 Q[NA][kC * kSB], K[NA][kC * kSB];
+  union {
+    struct {
+      float Us[10 * 16 * kST], Iv[4 * 16 * kST], In[10 * 16 * kST];
+    };
+    float core[kC * kSX];
+  };
+  __bf16 V[NA == 1 ? 8 : 1][NA == 1 ? kC * 16 : 1];  // bf16: each wave's columns of v
+  __device__ float& us(int i, int j) { return Us[PrepLds<true>::at(i, j)]; }
+  __device__ float& iv(int i, int j) { return Iv[(i >> 4) * (16 * kST) + (i & 15) * kST + (j & 15)]; }  // diagonal blocks
+};
+
+// x as the sum of three bf16 values (round to nearest each: the sum of the
+// first two is within 2^-17 of x, the three are exact but for f32 denormals)
+__device__ __forceinline__ void split3(const float* x, bf16x8* p) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    f32x2v r = {x[e], x[e + 1]};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const bf16x2v b = __builtin_convertvector(r, bf16x2v);
+      p[i][e] = b[0];
+      p[i][e + 1] = b[1];
+      r = r - __builtin_convertvector(b, f32x2v);
+    }
+  }
+}
+// acc += A . B over one 32-deep step: the parts' products whose order matters in f32
+template <int NA, int NB>
+__device__ __forceinline__ f32x4v mma_parts(const bf16x8* a, const bf16x8* b, f32x4v acc) {
+#pragma unroll
+  for (int o = (NA + NB - 2 < 2 ? NA + NB - 2 : 2); o >= 0; --o)
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+      if (o - i >= 0 && o - i < NB) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[o - i], acc, 0, 0, 0);
+  return acc;
+}
+
+typedef short s16x4v __attribute__((ext_vector_type(4)));
+
+// 16x16 diagonal block b of (I + L)^-1, L = Us strict lower, by forward
+// substitution: lane j (of each 16-lane group) owns column j, lane i keeps
+// row i of L, broadcast from its registers.
+template <typename LT>
+__device__ __forceinline__ void diag_inv(LT& L, int b, int lane) {
+  const int b0 = 16 * b, j = lane & 15;
+  f32x4 row[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) row[q] = *(const f32x4*)&L.us(b0 + j, b0 + 4 * q);
+  float col[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) col[k] = k == j ? 1.0f : 0.0f;
+#pragma unroll
+  for (int i = 1; i < 16; ++i) {
+    float acc[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < i; ++k) {
+      const float l = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, (float)row[k >> 2][k & 3]), i));
+      acc[k & 1] += l * col[k];
+    }
+    col[i] = i > j ? -(acc[0] + acc[1]) : col[i];
+  }
+  if (lane < 16) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) L.iv(b0 + i, b0 + j) = col[i];
+  }
+}
+
+// Raw buffer resource over `bytes` bytes at a wave-uniform address (moved to
+// SGPRs, where a resource must live).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(const void* p, int bytes) {
+  const uint64_t x = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)x), hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32));
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), (short)0, bytes, 0x00020000);
+}
+
+// 16 bytes a lane from the buffer into LDS at lds + 16 lane (lds wave-uniform).
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t src, void* lds, int offset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void*)lds, 16, offset, 0, 0, 0);
+}
+// Four bf16 values of one column in four rows (the transpose read).
+__device__ __forceinline__ bf16x4 read_tr(const __bf16* p) {
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4v*)p));
+}
+
+template <typename T>
+__global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2))) void gdn_fused_kernel(GdnArgs g) {
+  constexpr bool BF = sizeof(T) == 2;
+  constexpr int NA = FusedLds<T>::NA;
+  __shared__ FusedLds<T> L;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fm = lane & 15, fq = lane >> 4;
+  // consecutive items (the value heads of a key head, the heads of a row) on one XCD
+  const int n_items = gridDim.x;
+  const int item = n_items % kXcds == 0 ? (int)(blockIdx.x % kXcds) * (n_items / kXcds) + (int)(blockIdx.x / kXcds) : (int)blockIdx.x;
+  const int h = item % g.nv, r = item / g.nv, kh = h / (g.nv / g.nk);
+  const int key_dim = g.nk * kD, t_last = g.t - 1, col = 16 * wave + fm;
+  const T* cv = (const T*)g.conved + (int64_t)r * g.t * g.conv_dim;
+
+  // The chunk's inputs as loaded (clamped to the last token): q / k rows
+  // tid / 16 and + 32, 8 columns each, v in the accumulator layout, wave 0's
+  // gates.  The next chunk's load under this chunk's products.
+  const int i0 = tid >> 4, k8 = (tid & 15) * 8;
+  Raw8<T> qr[2], kr[2];
+  T ar, br;
+  float vr[BF ? 1 : 16];
+  const float dt_bias = g.dt_bias[h], neg_a = g.neg_a[h];
+  // slot s of a 16-row tile staged in LDS holds row 4 (s % 4) + s / 4, so
+  // that a read of rows 4 fq + e across the wave touches four slots in a row
+  auto slot_row = [](int s) { return 4 * (s & 3) + (s >> 2); };
+  auto load = [&](int t0) {
+    if (wave == 0) {
+      const int64_t ab = r * g.ab_sb + (int64_t)min(t0 + lane, t_last) * g.ab_st + h;
+      ar = ((const T*)g.a)[ab];
+      br = ((const T*)g.b)[ab];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const T* row = cv + (int64_t)min(t0 + i0 + 32 * u, t_last) * g.conv_dim;
+      qr[u].load(row + kh * kD + k8);
+      kr[u].load(row + key_dim + kh * kD + k8);
+    }
+    if constexpr (BF) {
+      // this wave's 16 columns of v by DMA: 32 rows of two 16-byte pieces each
+      const __amdgpu_buffer_rsrc_t rv = buffer_at(cv + 2 * key_dim + h * kD + 16 * wave, INT32_MAX);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int s = 32 * i + (lane >> 1);
+        const int t = min(t0 + 16 * (s >> 4) + slot_row(s & 15), t_last);
+        dma16(rv, L.V[wave] + 512 * i, t * g.conv_dim * 2 + 16 * (lane & 1));
+      }
+    } else {
+      const T* vcol = cv + 2 * key_dim + h * kD + col;
+#pragma unroll
+      for (int x = 0; x < 16; ++x) vr[x] = vcol[(int64_t)min(t0 + 16 * (x >> 2) + 4 * fq + (x & 3), t_last) * g.conv_dim];
+    }
+  };
+  load(0);
+  f32x4v S[8];
+  if (g.s_in) {
+    const float* sp = g.s_in + r * g.s_in_sb + (int64_t)h * kD * kD + col;
+#pragma unroll
+    for (int ti = 0; ti < 8; ++ti)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[ti][e] = sp[(16 * ti + 4 * fq + e) * kD];
+  } else {
+#pragma unroll
+    for (int ti = 0; ti < 8; ++ti) S[ti] = f32x4v{0, 0, 0, 0};
+  }
+
+  for (int c = 0; c < g.n_chunks; ++c) {
+    const int t0 = c * kC, left = g.t - t0;
+    const int nt = __builtin_amdgcn_readfirstlane(min(4, (left + 15) >> 4));  // row tiles with tokens
+    const bool have_state = c > 0 || g.s_in != nullptr;
+    if (c > 0) __syncthreads();  // the previous chunk's readers of L are done
+    // ---- gates (as in prep; cum one by one like the reference: a prefix scan
+    // over the lanes left the state five times further from 64 bits in f32,
+    // since e^(cum_i - cum_j) then sees two unrelated roundings)
+    if (wave == 0) {
+      const bool ok = t0 + lane < g.t;
+      const float x = to_f(ar) + dt_bias;
+      const float sp = fmaxf(x, 0.0f) + logf(expf(-fabsf(x)) + 1.0f);
+      const float gv = ok ? sp * neg_a : 0.0f;
+      float acc = 0.0f;
+#pragma unroll
+      for (int k = 0; k < kC; ++k) {
+        const float gk = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gv), k));
+        acc = acc + (k <= lane ? gk : 0.0f);
+      }
+      const float last = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), kC - 1));
+      L.betas[lane] = ok ? 1.0f / (1.0f + expf(-to_f(br))) : 0.0f;
+      L.cums[lane] = acc;
+      L.ecum[lane] = expf(acc);
+      L.ekd[lane] = expf(last - acc);
+      if (lane == 0) L.decay[0] = expf(last);
+    }
+    // ---- q and k as bf16 parts and their norms (zero past the last token)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bool ok = t0 + i0 + 32 * u < g.t;
+      float qv[8], kv[8];
+      float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        qv[e] = ok ? qr[u][e] : 0.0f;
+        kv[e] = ok ? kr[u][e] : 0.0f;
+        sq += qv[e] * qv[e];
+        sk += kv[e] * kv[e];
+      }
+      const float nq = sqrtf(row16_sum(sq) + 1e-6f), nk = sqrtf(row16_sum(sk) + 1e-6f);
+      const int at = (i0 + 32 * u) * kSB + k8;
+      bf16x8 qp[3], kp[3];
+      split3(qv, qp);
+      split3(kv, kp);
+#pragma unroll
+      for (int i = 0; i < NA; ++i) {
+        *(bf16x8*)(L.Q[i] + at) = qp[i];
+        *(bf16x8*)(L.K[i] + at) = kp[i];
+      }
+      if ((tid & 15) == 0) {
+        L.qf[i0 + 32 * u] = 0.08838834764831845f / nq;  // 128^-0.5
+        L.kf[i0 + 32 * u] = 1.0f / nk;
+      }
+    }
+    __syncthreads();
+
+    // ---- ut and intra tiles, the diagonal blocks' inverses (prep's split)
+    auto tile = [&](auto dg_c, auto dq_c, int ti, int tj) {
+      constexpr bool DG = decltype(dg_c)::value, DQ = decltype(dq_c)::value;
+      f32x4v ga = {0, 0, 0, 0}, qa = {0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < kD / 32; ++s) {
+        bf16x8 ki[NA], qi[NA], kj[NA];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+          const int a_at = (16 * ti + fm) * kSB + 32 * s + 8 * fq, b_at = (16 * tj + fm) * kSB + 32 * s + 8 * fq;
+          if (DG) ki[i] = *(const bf16x8*)(L.K[i] + a_at);
+          if (DQ) qi[i] = *(const bf16x8*)(L.Q[i] + a_at);
+          kj[i] = *(const bf16x8*)(L.K[i] + b_at);
+        }
+        if (DG) ga = mma_parts<NA, NA>(ki, kj, ga);
+        if (DQ) qa = mma_parts<NA, NA>(qi, kj, qa);
+      }
+      const int j = 16 * tj + fm;
+      const float kfj = L.kf[j], cj = L.cums[j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * ti + 4 * fq + e;
+        const float pair = j <= i ? expf(L.cums[i] - cj) : 0.0f;
+        if (DG) L.us(i, j) = j < i ? ga[e] * (L.betas[i] * L.kf[i]) * kfj * pair : 0.0f;
+        if (DQ) L.In[PrepLds<true>::at(i, j)] = j <= i ? qa[e] * L.qf[i] * kfj * pair : 0.0f;
+      }
+    };
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (wave < 3) {
+      // wave 0: (1,0) (2,0); wave 1: (2,1) (3,0); wave 2: (3,1) (3,2)
+      if (nt > (wave == 0 ? 1 : wave + 1)) tile(Yes{}, Yes{}, wave == 0 ? 1 : wave + 1, wave == 0 ? 0 : 1);
+      if (nt > (wave == 0 ? 2 : 3)) tile(Yes{}, Yes{}, wave == 0 ? 2 : 3, wave == 2 ? 2 : 0);
+    } else if (wave == 3) {
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (b < nt) tile(No{}, Yes{}, b, b);
+    } else if (wave - 4 < nt) {
+      tile(Yes{}, No{}, wave - 4, wave - 4);
+      wave_lds_sync();
+      diag_inv(L, wave - 4, lane);
+    }
+    // the norm's z rows load under the products
+    const int nrow = tid >> 3, c8 = 8 * (tid & 7), nt_row = t0 + nrow;
+    const bool row_ok = nt_row < g.t;
+    const T* zr = (const T*)g.z + r * g.z_sb + (int64_t)min(nt_row, t_last) * g.z_st + h * kD;
+    T* yr = (T*)g.y + r * g.y_sb + (int64_t)min(nt_row, t_last) * g.y_st + h * kD;
+    float z[2][8];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) load_channels<T, 1>(zr + 64 * k + c8, g.norm_vec, z[k]);
+    // ---- ks = k S and qs = q S over this wave's columns, in four K steps of 32
+    f32x4v ks[4], qs[4];
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) ks[ti] = qs[ti] = f32x4v{0, 0, 0, 0};
+    auto state_step = [&](auto s_c) {
+      constexpr int s = decltype(s_c)::value;
+      if (!have_state) return;
+      const float x[8] = {S[2 * s][0], S[2 * s][1], S[2 * s][2], S[2 * s][3], S[2 * s + 1][0], S[2 * s + 1][1], S[2 * s + 1][2], S[2 * s + 1][3]};
+      bf16x8 sp[3];
+      split3(x, sp);
+      auto rows = [&](const __bf16* m, int ti) {
+        const __bf16* p = m + (16 * ti + fm) * kSB + 32 * s + 4 * fq;
+        const bf16x4 lo = *(const bf16x4*)p, hi = *(const bf16x4*)(p + 16);
+        return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      };
+#pragma unroll
+      for (int ti = 0; ti < 4; ++ti) {
+        if (ti >= nt) break;
+        bf16x8 a[NA];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) a[i] = rows(L.K[i], ti);
+        ks[ti] = mma_parts<NA, 3>(a, sp, ks[ti]);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) a[i] = rows(L.Q[i], ti);
+        qs[ti] = mma_parts<NA, 3>(a, sp, qs[ti]);
+      }
+    };
+    state_step(std::integral_constant<int, 0>{});
+    state_step(std::integral_constant<int, 1>{});
+    state_step(std::integral_constant<int, 2>{});
+    state_step(std::integral_constant<int, 3>{});
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's v is in LDS
+    __syncthreads();  // ut, the diagonal inverses and intra are in LDS
+
+    // ---- v_new, out and the state update: this wave's columns only
+    f32x4v vn[4], out[4];
+    auto v_at = [&](int ti, int e) {
+      if constexpr (BF)
+        return (float)L.V[wave][16 * (16 * ti + 4 * e + fq) + fm];
+      else
+        return vr[4 * ti + e];
+    };
+    // (I + ut) v_new = w by block forward substitution: the accumulator layout
+    // is the B operand of the next product (K slot fq, step e: row 4 fq + e)
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      vn[ti] = f32x4v{0, 0, 0, 0};
+      if (ti >= nt) continue;
+      const f32x4 b4 = *(const f32x4*)(L.betas + 16 * ti + 4 * fq), e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq);
+      const f32x4 k4 = *(const f32x4*)(L.kf + 16 * ti + 4 * fq);
+      f32x4v lv = {0, 0, 0, 0};
+#pragma unroll
+      for (int tj = 0; tj < ti; ++tj) {
+        const f32x4 a4 = *(const f32x4*)&L.us(16 * ti + fm, 16 * tj + 4 * fq);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lv = mma16(a4[e], vn[tj][e], lv);
+      }
+      const f32x4 a4 = *(const f32x4*)&L.iv(16 * ti + fm, 16 * ti + 4 * fq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool ok = t0 + 16 * ti + 4 * fq + e < g.t;
+        const float w = b4[e] * ((ok ? v_at(ti, e) : 0.0f) - e4[e] * (k4[e] * ks[ti][e])) - lv[e];
+        vn[ti] = mma16(a4[e], w, vn[ti]);
+      }
+    }
+    if (c + 1 < g.n_chunks) load(t0 + kC);
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      const f32x4 e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq), q4 = *(const f32x4*)(L.qf + 16 * ti + 4 * fq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[ti][e] = e4[e] * (q4[e] * qs[ti][e]);
+      if (ti >= nt) continue;
+#pragma unroll
+      for (int tj = 0; tj <= ti; ++tj) {
+        const f32x4 a4 = *(const f32x4*)&L.In[PrepLds<true>::at(16 * ti + fm, 16 * tj + 4 * fq)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[ti] = mma16(a4[e], vn[tj][e], out[ti]);
+      }
+    }
+    {
+      const float decay = L.decay[0];
+#pragma unroll
+      for (int ti = 0; ti < 8; ++ti) S[ti] = S[ti] * decay;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if (2 * p >= nt) break;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const f32x4 k4 = *(const f32x4*)(L.kf + 32 * p + 16 * j + 4 * fq), d4 = *(const f32x4*)(L.ekd + 32 * p + 16 * j + 4 * fq);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[4 * j + e] = vn[2 * p + j][e] * k4[e] * d4[e];
+        }
+        bf16x8 xp[3];
+        split3(x, xp);
+        // k^T: four tokens of column 16 ti + fm per transpose read
+        const int row = 32 * p + 4 * fq + (fm >> 2);
+#pragma unroll
+        for (int ti = 0; ti < 8; ++ti) {
+          bf16x8 a[NA];
+#pragma unroll
+          for (int i = 0; i < NA; ++i) {
+            const __bf16* kp = L.K[i] + row * kSB + 16 * ti + 4 * (fm & 3);
+            const bf16x4 lo = read_tr(kp), hi = read_tr(kp + 16 * kSB);
+            a[i] = bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          }
+          S[ti] = mma_parts<NA, 3>(a, xp, S[ti]);
+        }
+      }
+    }
+
+    // ---- gated norm of the chunk's rows: 8 threads a row, 16 columns each
+    __syncthreads();  // everyone is done with the tiles that core lies over
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) L.core[(16 * ti + 4 * fq + e) * kSX + col] = out[ti][e];
+    __syncthreads();
+    float o[2][8];
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      load8<float>(L.core + nrow * kSX + 64 * k + c8, o[k]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum += o[k][e] * o[k][e];
+    }
+    sum += dpp_f<0xB1>(sum);
+    sum += dpp_f<0x4E>(sum);
+    sum += dpp_f<0x141>(sum);
+    const float inv = 1.0f / sqrtf(sum / (float)kD + g.eps);
+    if (row_ok) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        float wv[8], y[8];
+        load_channels<float, 1>(g.norm_w + 64 * k + c8, g.norm_vec, wv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = gated_norm(o[k][e], inv, wv[e], z[k][e]);
+        if (g.norm_vec) {
+          store8<T>(yr + 64 * k + c8, y);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) yr[64 * k + c8 + e] = from_f<T>(y[e]);
+        }
+      }
+    }
+  }
+  float* const so = g.s_out + (int64_t)item * kD * kD + col;
+#pragma unroll
+  for (int ti = 0; ti < 8; ++ti)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) so[(16 * ti + 4 * fq + e) * kD] = S[ti][e];
+}
+
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct GdnLayout {
@@ -1268,6 +1660,22 @@ GdnLayout gdn_layout(const cev_gdn_desc* d) {
   L.core = L.rec + align256((size_t)d->batch * d->n_v_heads * n_chunks * kRecFloats * sizeof(float));
   L.total = L.core + align256((size_t)d->batch * d->t * d->n_v_heads * d->head_v_dim * sizeof(float));
   return L;
+}
+
+// Whether the fused kernel runs a call, by modelled times in us that fit 32
+// traced calls (1-32 rows of 1-4096 tokens, both dtypes): the fused kernel
+// takes one workgroup a CU and 14 (f32: 20) a chunk; prep, scan and norm
+// launch apart, prep works on every chunk at once and the scan on eight
+// 16-column slices of each head at once, which wins for few long rows (one
+// bf16 row of 4096 tokens: 317 against 885).  One chunk is always fused.
+bool use_fused(const GdnArgs& g, bool bf) {
+  // v's buffer offsets are 32-bit; one chunk cannot come near that
+  if (g.n_chunks == 1) return true;
+  if ((int64_t)g.t * g.conv_dim * 2 > INT32_MAX) return false;
+  const double items = (double)g.batch * g.nv, n = g.n_chunks, cus = kConvCus;
+  const double fused = std::ceil(items / cus) * n * (bf ? 14.0 : 20.0);
+  const double apart = 15.0 + items * n * (bf ? 0.039 : 0.083) + std::ceil(items * (kD / kW) / cus) * n * (bf ? 3.3 : 3.0);
+  return fused < apart;
 }
 
 int32_t check_gdn(const cev_gdn_desc* d) {
@@ -1388,35 +1796,38 @@ extern "C" int32_t cev_gdn_forward(const cev_gdn_desc* d, const void* mixed, con
   const int64_t conv_items = (int64_t)g.batch * ((g.t + kConvRunLong - 1) / kConvRunLong) * (g.conv_dim / 8);
   const bool long_runs = conv_items >= 2 * (int64_t)kConvCus * kConvThreads;
   const int64_t recs = (int64_t)g.batch * g.nv * g.n_chunks;
-  // scan grid: (bf16, many chunks) groups of value heads per key head, rounded up to the 8 XCDs, x group size x slices
-  const int64_t grp = d->dtype == CEV_BF16 && g.n_chunks > 1 ? g.nv / g.nk : 1;
+  // scan grid: (bf16) groups of value heads per key head, rounded up to the 8 XCDs, x group size x slices
+  const int64_t grp = d->dtype == CEV_BF16 ? g.nv / g.nk : 1;
   const int64_t slices = ((int64_t)g.batch * g.nv / grp + kXcds - 1) / kXcds * kXcds * grp * (kD / kW);
   const int64_t norm_items = (int64_t)g.batch * g.t * g.nv;
   if (recs > INT32_MAX || (int64_t)g.batch * ((g.t + kConvRunShort - 1) / kConvRunShort) * ((g.conv_dim / 8 + kConvThreads - 1) / kConvThreads) > INT32_MAX) return cev_fail(CEV_ERR_UNSUPPORTED, "GDN grid too large");
-  if (d->dtype == CEV_BF16) {
-    launch_conv<__bf16>(g, long_runs, s);
-    hipLaunchKernelGGL(gdn_prep_kernel<__bf16>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
-  } else {
-    launch_conv<float>(g, long_runs, s);
-    hipLaunchKernelGGL(gdn_prep_kernel<float>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
-  }
-  const bool bf = d->dtype == CEV_BF16;
-  if (g.n_chunks > 1) {
-    if (bf)
-      hipLaunchKernelGGL(gdn_scan_kernel<true>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
-    else
-      hipLaunchKernelGGL(gdn_scan_kernel<false>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
-  } else {
-    if (bf)
-      hipLaunchKernelGGL(gdn_scan_one_chunk_kernel<true>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
-    else
-      hipLaunchKernelGGL(gdn_scan_one_chunk_kernel<false>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
-  }
-  // 16-byte aligned rows of z and y (and norm_w) for the vector norm
   const int64_t vec = d->dtype == CEV_BF16 ? 8 : 4;
-  const bool norm_vec = ((uintptr_t)g.z | (uintptr_t)g.y | (uintptr_t)g.norm_w) % 16 == 0 && g.z_sb % vec == 0 && g.z_st % vec == 0 &&
-                        g.y_sb % vec == 0 && g.y_st % vec == 0;
-  if (norm_vec) {
+  // 16-byte aligned rows of z and y (and norm_w) for the vector norm
+  g.norm_vec = ((uintptr_t)g.z | (uintptr_t)g.y | (uintptr_t)g.norm_w) % 16 == 0 && g.z_sb % vec == 0 && g.z_st % vec == 0 &&
+               g.y_sb % vec == 0 && g.y_st % vec == 0;
+  if (d->dtype == CEV_BF16)
+    launch_conv<__bf16>(g, long_runs, s);
+  else
+    launch_conv<float>(g, long_runs, s);
+  if (use_fused(g, d->dtype == CEV_BF16)) {
+    const dim3 grid((unsigned)(g.batch * g.nv));
+    if (d->dtype == CEV_BF16)
+      hipLaunchKernelGGL(gdn_fused_kernel<__bf16>, grid, dim3(kPrepThreads), 0, s, g);
+    else
+      hipLaunchKernelGGL(gdn_fused_kernel<float>, grid, dim3(kPrepThreads), 0, s, g);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return cev_fail(CEV_ERR_HIP, "GDN launch: %s", hipGetErrorString(e));
+    return CEV_OK;
+  }
+  if (d->dtype == CEV_BF16)
+    hipLaunchKernelGGL(gdn_prep_kernel<__bf16>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
+  else
+    hipLaunchKernelGGL(gdn_prep_kernel<float>, dim3((unsigned)recs), dim3(kPrepThreads), 0, s, g);
+  if (d->dtype == CEV_BF16)
+    hipLaunchKernelGGL(gdn_scan_kernel<true>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
+  else
+    hipLaunchKernelGGL(gdn_scan_kernel<false>, dim3((unsigned)slices), dim3(kScanThreads), 0, s, g);
+  if (g.norm_vec) {
     const dim3 grid((unsigned)((norm_items + 16 * kNormRows - 1) / (16 * kNormRows)));
     if (d->dtype == CEV_BF16)
       hipLaunchKernelGGL(gdn_norm_vec_kernel<__bf16>, grid, dim3(256), 0, s, g);

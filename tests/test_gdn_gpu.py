@@ -396,3 +396,29 @@ def test_conv_on_unaligned_views(gpu, bf16, t):
         assert torch.equal(x, y)
     seq = torch.cat([s1, mixed.transpose(1, 2)], 2)
     assert torch.equal(got[1], seq[:, :, t:])
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("batch,t,state", [(1, 1, True), (2, 15, False), (1, 16, True), (3, 17, True), (2, 33, False), (2, 48, True), (1, 49, True),
+                                           (5, 64, True), (9, 65, True), (9, 130, False)])
+def test_fused_rows_vs_oracle(gpu, orc, bf16, batch, t, state):
+    """The one-kernel path at the edges of its 16-row tiles and 64-token
+    chunks, with and without a state, against the oracle layer (which works
+    chunk by chunk with explicit inverses)."""
+    w = configs.GdnWorkload("gdn-fused", 21 + t, bf16, batch, t, nk=2, nv=4)
+    inp = w.inputs()
+    rng = np.random.default_rng(t)
+    kw_d, kw_o = {}, {}
+    if state:
+        conv_in = rng.standard_normal((batch, w.conv_dim, 3)).astype(np.float32)
+        s_in = (0.1 * rng.standard_normal((batch, 4, 128, 128))).astype(np.float32)
+        if bf16:
+            conv_in = cev_hip.synth.round_bf16(conv_in)
+        kw_o = dict(conv_in=conv_in, s_in=s_in)
+        kw_d = dict(conv_in=to_dev(conv_in, bf16, gpu), s_in=to_dev(s_in, False, gpu))
+    y, co, so = _run_gpu(w, inp, gpu, **kw_d)
+    ry, rco, rso = _run_oracle(orc, w, inp, **kw_o)
+    ey, es = float(np.abs(to_np(y) - ry).max()), float(np.abs(to_np(so) - rso).max())
+    _say(f"fused {batch} x {t} bf16={bf16} state={state}: max|d| y {ey:.3g} state {es:.3g}")
+    assert np.array_equal(to_np(co), rco)
+    assert es <= F32_TOL and ey <= (BF16_TOL if bf16 else F32_TOL)
