@@ -1426,6 +1426,18 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
       }
       const float nq = sqrtf(row16_sum(sq) + 1e-6f), nk = sqrtf(row16_sum(sk) + 1e-6f);
       const int at = (i0 + 32 * u) * kSB + k8;
+      if constexpr (!BF) {
+        // f32 models: the rows themselves are normalised (one rounding less
+        // than a factor applied later); the factors are then 1.  x / n as
+        // x * (1/n) and one correction: rounded like the division.
+        const float rq = 1.0f / nq, rk = 1.0f / nk;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float a = qv[e] * rq, b = kv[e] * rk;
+          qv[e] = __builtin_fmaf(__builtin_fmaf(-a, nq, qv[e]), rq, a) * 0.08838834764831845f;
+          kv[e] = __builtin_fmaf(__builtin_fmaf(-b, nk, kv[e]), rk, b);
+        }
+      }
       bf16x8 qp[3], kp[3];
       split3(qv, qp);
       split3(kv, kp);
@@ -1435,8 +1447,8 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
         *(bf16x8*)(L.K[i] + at) = kp[i];
       }
       if ((tid & 15) == 0) {
-        L.qf[i0 + 32 * u] = 0.08838834764831845f / nq;  // 128^-0.5
-        L.kf[i0 + 32 * u] = 1.0f / nk;
+        L.qf[i0 + 32 * u] = BF ? 0.08838834764831845f / nq : 1.0f;  // 128^-0.5
+        L.kf[i0 + 32 * u] = BF ? 1.0f / nk : 1.0f;
       }
     }
     __syncthreads();
