@@ -118,6 +118,247 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_rows_kernel(LinArgs a) 
   }
 }
 
+// ---------------------------------------------------------------------------
+// f32 products of more than kRowsSmall rows on the bf16 matrix cores.
+// Every f32 value is split into three bf16 parts (round to nearest each; the
+// parts' sum is the value) and six of the nine part products are summed in
+// f32: the three dropped ones are below 2^-26 of the product each.  Six bf16
+// products cost 6/16 of the f32 unit's time, and the accumulator is rounded
+// once per 16 products of a part pair instead of once per 2.
+//
+// A workgroup of eight waves computes a 128 x 128 tile of y, each wave 64 x 32
+// of it on 32x32x16 MFMAs.  A 32-deep slice of x and w goes through registers
+// two slices ahead, is split there once for the whole workgroup while the
+// slice before it is multiplied, and lies in LDS (two buffers of 48 KB) as
+// three planes of 64-byte rows, 16-byte piece c of row r at c ^ (r / 4 % 4) so
+// that a fragment read touches every bank.
+// What bounds it: a slice takes 3000 clocks a CU where its MFMAs need 1536 and
+// its LDS traffic (195 KB) 1500; 185-193 TFLOP/s of f32 products at 2048 rows
+// (library 131-149).  Tried: one buffer and one slice ahead 134 us at
+// 200 x 4096 x 2048 (72 now); four waves a tile 89; 64-wide tiles 113 against
+// 95 at 912 x 4096 x 2048; 256 x 128 tiles 4-6 % faster at 2048 rows and half
+// a round short at 912.
+// Error against f64, N(0,1) x 0.02 N(0,1): 7.0e-7 at k = 2048 (library
+// 8.1e-7), 1.24e-6 at 6144 (1.40e-6).
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kSliceK = 32;
+
+constexpr int kSplitTile = 128, kSplitWaves = 8;
+
+__global__ __launch_bounds__(kSplitWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void linear_split_kernel(LinArgs a, int parts) {
+  constexpr int BM = kSplitTile, BN = kSplitTile, RP = kSplitWaves * 8;  // RP: rows per pass of the workgroup's loads
+  constexpr int WM = BM / 2, WN = BN / (kSplitWaves / 2), TM = WM / 32, TN = WN / 32;
+  constexpr int NX = BM / RP, NW = BN / RP;         // 16-byte loads per thread and slice
+  constexpr int kPlane = (BM + BN) * kSliceK;       // one part of both operands, in bf16 values
+  constexpr int kBuf = 3 * kPlane;                  // one slice
+  __shared__ __align__(16) __bf16 lds[2 * kBuf];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n32 = lane & 31, u = lane >> 5, wm = wave & 1, wn = wave >> 1;
+  // tiles of one XCD (workgroups go round-robin over the 8) are neighbours, m
+  // fastest: they share w's rows
+  const int total = gridDim.x, q8 = total / 8, r8 = total % 8, xcd = blockIdx.x % 8;
+  const int mt = (int)((a.m + BM - 1) / BM), tiles = total / parts;
+  int id = xcd * q8 + min(xcd, r8) + blockIdx.x / 8;
+  const int part = id / tiles;
+  id -= part * tiles;
+  const int m0 = (id % mt) * BM, n0 = (id / mt) * BN;
+
+  // this thread's rows (clamped) and column of a slice
+  const int row = tid >> 3, c4 = (tid & 7) * 4;
+  const float* xp[NX];
+  const float* wp[NW];
+#pragma unroll
+  for (int i = 0; i < NX; ++i) xp[i] = (const float*)a.x + (int64_t)min(m0 + row + RP * i, (int)a.m - 1) * a.ldx;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) wp[i] = (const float*)a.w + (int64_t)min(n0 + row + RP * i, (int)a.n - 1) * a.ldw;
+  f32x4 xr[2][NX], wr[2][NW];  // two slices on their way
+  auto load = [&](int k0, f32x4* xr, f32x4* wr) {
+    // columns past k read the row's last four and count as zero
+    const int k = k0 + c4, kc = min(k, (int)a.k - 4);
+    const bool ok = k < (int)a.k;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const f32x4 v = *(const f32x4*)(xp[i] + kc);
+      xr[i] = ok ? v : f32x4{0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const f32x4 v = *(const f32x4*)(wp[i] + kc);
+      wr[i] = ok ? v : f32x4{0, 0, 0, 0};
+    }
+  };
+  // row r of a plane (x's rows, then w's), 4 values at column c4
+  auto put = [&](int buf, int r, const f32x4& v) {
+    const int at = buf * kBuf + r * kSliceK + ((((c4 >> 3) ^ (r >> 2)) & 3) << 3) + (c4 & 4);
+    f32x2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const bf16x2 a2 = __builtin_convertvector(lo, bf16x2), b2 = __builtin_convertvector(hi, bf16x2);
+      *(bf16x4*)(lds + i * kPlane + at) = bf16x4{a2[0], a2[1], b2[0], b2[1]};
+      lo -= __builtin_convertvector(a2, f32x2);
+      hi -= __builtin_convertvector(b2, f32x2);
+    }
+  };
+  auto frag = [&](int buf, int plane, int r, int ks) {
+    return *(const bf16x8*)(lds + buf * kBuf + plane * kPlane + r * kSliceK + ((((2 * ks + u) ^ (r >> 2)) & 3) << 3));
+  };
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+  // this part's slices of k
+  const int all = (int)((a.k + kSliceK - 1) / kSliceK);
+  const int s0 = (int)((int64_t)part * all / parts), s1 = (int)((int64_t)(part + 1) * all / parts);
+  auto put_x = [&](int buf, const f32x4* v) {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) put(buf, row + RP * i, v[i]);
+  };
+  auto put_w = [&](int buf, const f32x4* v) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) put(buf, BM + row + RP * i, v[i]);
+  };
+  auto multiply = [&](int buf, int ks) {
+    bf16x8 fx[TM][3], fw[TN][3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) fx[i][p] = frag(buf, p, wm * WM + 32 * i + n32, ks);
+#pragma unroll
+      for (int j = 0; j < TN; ++j) fw[j][p] = frag(buf, p, BM + wn * WN + 32 * j + n32, ks);
+    }
+    // small products first
+#pragma unroll
+    for (int o = 2; o >= 0; --o)
+#pragma unroll
+      for (int p = 0; p <= o; ++p)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i][p], fw[j][o - p], acc[i][j], 0, 0, 0);
+  };
+  // Slice sl is multiplied while slice sl + 1 is split into the other buffer
+  // (past the end: a repeat of the last columns, counted as zero) and slices
+  // sl + 2 and sl + 3 load.
+  auto step = [&](int sl, auto buf_c) {
+    constexpr int B = decltype(buf_c)::value, N = B ^ 1;
+    multiply(B, 0);
+    put_x(N, xr[N]);
+    multiply(B, 1);
+    put_w(N, wr[N]);
+    load((sl + 3) * kSliceK, xr[N], wr[N]);
+    __syncthreads();
+  };
+  load(s0 * kSliceK, xr[0], wr[0]);
+  load((s0 + 1) * kSliceK, xr[1], wr[1]);
+  put_x(0, xr[0]);
+  put_w(0, wr[0]);
+  load((s0 + 2) * kSliceK, xr[0], wr[0]);
+  __syncthreads();
+  for (int sl = s0; sl < s1; sl += 2) {
+    step(sl, std::integral_constant<int, 0>{});
+    if (sl + 1 < s1) step(sl + 1, std::integral_constant<int, 1>{});
+  }
+
+  // An infinite value (or one above bf16's range) has no parts: x - bf16(x) is
+  // not a number.  A wave whose quarter came out non-finite anywhere computes
+  // it again in f32, one product after the other.
+  float worst = 0.0f;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) worst += acc[i][j][e] * 0.0f;
+  float* y = (float*)a.y + (int64_t)part * a.m * a.ldy;  // parts lie behind one another
+  const int k0 = s0 * kSliceK, k1 = min(s1 * kSliceK, (int)a.k);
+  if (__builtin_expect(__any(worst != 0.0f || worst != worst) != 0, 0)) {
+#pragma unroll 1
+    for (int e = lane; e < WM * WN; e += 64) {
+      const int m = m0 + wm * WM + e / WN, n = n0 + wn * WN + e % WN;
+      if (m >= a.m || n >= a.n) continue;
+      const float* xq = (const float*)a.x + (int64_t)m * a.ldx;
+      const float* wq = (const float*)a.w + (int64_t)n * a.ldw;
+      float s = 0.0f;
+#pragma unroll 1
+      for (int k = k0; k < k1; ++k) s = __builtin_fmaf(xq[k], wq[k], s);
+      y[(int64_t)m * a.ldy + n] = s * a.alpha;
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * WN + 32 * j + n32;
+    if (n >= a.n) continue;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm * WM + 32 * i + 8 * (e >> 2) + 4 * u + (e & 3);
+        if (m < a.m) y[(int64_t)m * a.ldy + n] = acc[i][j][e] * a.alpha;
+      }
+  }
+}
+
+// y = alpha * the sum of the parts (f32, part after part).
+__global__ __launch_bounds__(256) void linear_parts_kernel(const float* ws, LinArgs a, int parts) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4, total = a.m * a.n;
+  if (i >= total) return;
+  f32x4 v = *(const f32x4*)(ws + i);
+  for (int p = 1; p < parts; ++p) v += *(const f32x4*)(ws + p * total + i);
+  // n is a multiple of 4 here, so the four values are one row's
+  const int64_t r = total <= UINT32_MAX ? (int64_t)((uint32_t)i / (uint32_t)a.n) : i / a.n;
+  *(f32x4*)((float*)a.y + r * a.ldy + (i - r * a.n)) = v * a.alpha;
+}
+
+// Parts of k for the split kernel (0: the library's f32 product), by modelled
+// times in us: a slice of a 128 x 128 tile takes a CU 1.1, 1.4 when all CUs
+// work (the clock drops), tiles x parts run in rounds of 256, parts are summed
+// by one more pass; the library reaches about 120 TFLOP/s on the f32 unit.
+// The new form has to win by 5 %.  Measured, library -> this (m x n x k):
+//   912 x 4096 x 2048 137 -> 95 us, 912 x 12288 x 2048 355 -> 268,
+//   2048 x 4096 x 2048 261 -> 187, 2048 x 2048 x 6144 346 -> 267;
+//   200 x 4096 x 2048 (64 tiles) 39 against 72 stays with the library.
+int split_parts(const LinArgs& a, size_t ws_bytes) {
+  constexpr int kCus = 256;
+  const int64_t tiles = ((a.m + kSplitTile - 1) / kSplitTile) * ((a.n + kSplitTile - 1) / kSplitTile);
+  if (a.m < kSplitTile || tiles > (1 << 24)) return 0;
+  const double slices = std::ceil((double)a.k / kSliceK);
+  double best = 0.95 * (8.0 + 2.0 * (double)a.m * (double)a.n * (double)a.k / 120e6);
+  int parts = 0;
+  for (int p = 1; p <= 4; p *= 2) {
+    const size_t bytes = (size_t)p * a.m * a.n * 4;
+    if (p > 1 && (bytes > ws_bytes || a.n % 4 != 0 || slices < 16 * p)) break;
+    const int64_t wgs = tiles * p;
+    double us = 6.0 + std::ceil(slices / p) * ((double)(wgs / kCus) * 1.4 + (wgs % kCus ? 1.1 : 0.0));
+    if (p > 1) us += 4.0 + (double)(bytes + a.m * a.n * 4) / 4e6;
+    if (us < best) {
+      best = us;
+      parts = p;
+    }
+  }
+  return parts;
+}
+
+int32_t launch_split(const LinArgs& a, int parts, void* ws, hipStream_t s) {
+  const int64_t grid = ((a.m + kSplitTile - 1) / kSplitTile) * ((a.n + kSplitTile - 1) / kSplitTile) * parts;
+  LinArgs b = a;
+  if (parts > 1) {
+    b.y = ws;
+    b.ldy = a.n;
+    b.alpha = 1.0f;
+  }
+  hipLaunchKernelGGL(linear_split_kernel, dim3((unsigned)grid), dim3(kSplitWaves * 64), 0, s, b, parts);
+  if (parts > 1)
+    hipLaunchKernelGGL(linear_parts_kernel, dim3((unsigned)((a.m * a.n / 4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, a, parts);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return cev_fail(CEV_ERR_HIP, "cev_linear launch: %s", hipGetErrorString(e));
+  return CEV_OK;
+}
+
 struct GatherArgs {
   const void* table;
   const int32_t* ids;
@@ -360,6 +601,11 @@ extern "C" int32_t cev_linear(cev_blas handle, int32_t dtype, int32_t out_dtype,
                 kRowsSmall, ovec);
   CEV_CHECK_ARG(handle != nullptr, "cev_linear: more than %d rows need a cev_blas handle", kRowsSmall);
   CEV_CHECK_ARG(workspace_bytes == 0 || workspace != nullptr, "cev_linear: null workspace of %zu bytes", workspace_bytes);
+  if (dtype == CEV_F32) {
+    const LinArgs a{x, w, y, m, n, k, ldx, ldw, ldy, alpha};
+    const int parts = split_parts(a, aligned16(workspace) ? workspace_bytes : 0);
+    if (parts > 0) return launch_split(a, parts, workspace, s);
+  }
   Blas* b = (Blas*)handle;
   std::lock_guard<std::mutex> lock(b->mu);
   GemmPlan* p = nullptr;

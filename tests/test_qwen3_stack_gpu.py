@@ -338,3 +338,45 @@ def test_debias_position_invariant_model_and_invalid_spans(gpu):
     dup[begin[2] + 1, :8] = [0, 0, 2, 3, 4, 5, 6, 7]
     got = _device_debias(gpu, logits, dup, begin, length, kk)
     assert np.isnan(got[2, :8]).all() and np.isfinite(got[0, :5]).all() and np.isfinite(got[1, :2]).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 12288, 2048), (129, 12300, 2044), (200, 12288, 36), (912, 2048, 6144), (1000, 4095, 516),
+                                   (2050, 4096, 128), (1300, 2048, 2048)])
+def test_split_f32_product(gpu, m, n, k):
+    """f32 products on the bf16 matrix cores: remainders of the 128-wide tiles
+    and of the 32-deep slices (k = 36: two slices, most loads past the end),
+    one part of k and several, against f64.  An output is a sum of k products;
+    16 of them share an f32 rounding of each of the six part pairs, so its error is within
+    6 (k / 16 + 16) 2^-24 of sum |x| |w|, and dropped part products add 3 2^-26."""
+    import torch
+
+    import cev_hip
+    g = torch.Generator().manual_seed(m + k)
+    x, w = torch.randn(m, k, generator=g).to(gpu), torch.randn(n, k, generator=g).to(gpu)
+    ld = n + 4 - n % 4 if n % 4 else n
+    out = torch.full((m, ld), float("nan"), device=gpu)[:, :n]
+    got = cev_hip.linear(x, w, out=out, alpha=0.5).double()
+    want = 0.5 * x.double() @ w.double().t().contiguous()
+    bound = 0.5 * ((k / 16 + 16) * 2.0**-24 + 3 * 2.0**-26) * (x.double().abs() @ w.double().abs().t().contiguous()) * 6
+    assert ((got - want).abs() <= bound).all()
+    assert (got - want).norm() / want.norm() < 3e-6
+
+
+def test_split_f32_product_keeps_infinities(gpu):
+    """Values without bf16 parts (infinite, or above bf16's range) give what
+    plain f32 products give: their tile is computed again one by one."""
+    import torch
+
+    import cev_hip
+    m, n, k = 256, 12288, 64
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+    x[3, 5], x[40, 7], x[200, 0], w[900, 9] = float("inf"), 3.4e38, float("nan"), -float("inf")
+    w[:, 7] = 1e-30
+    got = cev_hip.linear(x.to(gpu), w.to(gpu)).cpu()
+    want = x.double() @ w.double().t()
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), fin)
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)].float())
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.allclose(got[fin].double(), want[fin], rtol=1e-4, atol=1e-4)
