@@ -380,3 +380,22 @@ def test_split_f32_product_keeps_infinities(gpu):
     assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)].float())
     assert torch.equal(torch.isnan(got), torch.isnan(want))
     assert torch.allclose(got[fin].double(), want[fin], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dt,odt", [("bf16", "bf16"), ("bf16", "f32"), ("f32", "bf16"), ("f32", "f32")])
+@pytest.mark.parametrize("width,off", [(8, 0), (2048, 0), (2056, 0), (2048, 1), (12, 0), (7, 0)])
+def test_gather_rows_forms(gpu, dt, odt, width, off):
+    """Wide and element-wise gathers (odd widths, unaligned views) give the
+    same rows, and an index outside the table a NaN row."""
+    import torch
+
+    import cev_hip
+    T, O = (torch.bfloat16 if d == "bf16" else torch.float32 for d in (dt, odt))
+    base = torch.randn(50, width + off, generator=torch.Generator().manual_seed(width)).to(T).to(gpu)
+    table = base[:, off:]
+    ids = torch.tensor([0, 49, 7, -1, 50, 7], dtype=torch.int32, device=gpu)
+    got = cev_hip.gather_rows(table, ids, out_dtype=O)
+    want = table[[0, 49, 7, 0, 0, 7]].to(O)
+    assert torch.equal(got[[0, 1, 2, 5]], want[[0, 1, 2, 5]])
+    assert got[3:5].isnan().all()
+    assert torch.equal(cev_hip.gather_rows(table, out_dtype=O), table.to(O))
