@@ -250,10 +250,9 @@ constexpr int32_t kMinFullLocal = 128;
 
 // Whether the small-launch kernel (a workgroup per 32 query slots, keys split
 // over its kFanWaves waves) runs this plan, by modelled times in us of both
-// forms.  The constants are fits to kernel traces of 60 launches (1-63
+// forms.  The constants are fits to kernel traces of 80 launches (1-63
 // blocks of 8-96 rows after 0-32k keys and 1-16 bidirectional rows; 4 to
-// 256 workgroups of the 256-slot kernels), most within 15 % and none chosen
-// wrongly by more than 2 us:
+// 256 workgroups of the 256-slot kernels), most within 15 %:
 //   256-slot kernels: base + per-chunk time (it grows with the share f of
 //     busy slots) x chunks of the longest part x rounds of 256 workgroups, a
 //     gated epilogue where no merge carries it, and the merge by its bytes;
@@ -288,7 +287,7 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
                                 (double)(all_chunks * d->n_kv_heads) / kSplitTargetWorkgroups);
   double whole = merge_us(p.n_splits);
   if (!bf)
-    whole += 8.0 + steps * (f > 0.5 ? 8.2 : 4.2);
+    whole += 8.0 + steps * (f > 0.5 ? 8.2 : 4.6);
   else if (wide)
     whole += 14.0 + steps * (0.9 + 0.9 * f) + (d->has_gate && p.n_splits == 1 ? 17.0 * f : 0.0);
   else
@@ -326,7 +325,7 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
     const double r = (double)max_rounds, avg = (double)sum_rounds / (double)n_subs;
     double us = merge_us(parts);
     if (!bf)
-      us += 6.0 + 5.2 * std::max(r, cu_rounds * avg);
+      us += 3.0 + std::max(8.0 + 4.0 * r, cu_rounds * (8.0 + 4.0 * avg));
     else if (wide)
       us += 3.0 + std::max(10.0 + 2.0 * r, cu_rounds * (10.0 + 2.0 * avg));
     else

@@ -1589,7 +1589,8 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel_wide(AttnArgs a) 
 //   bf16 d = 128: 1 x 19 tokens after 301 keys 15.0 -> 9.5 us, 8 x 61-77
 //   after 74 25.5 -> 11.6, 11 x 21-44 after 421 31.4 -> 16.6;
 //   bf16 d = 256 gated: 5 rows of 43 40.0 -> 14.7, 4 x 28-40 after 123
-//   42.6 -> 16.2;  f32: 5 x 33-43 after 47 31.2 -> 13.9.
+//   42.6 -> 16.2;  f32: 5 x 33-43 after 47 31.2 -> 14.2, 12 x 32 after 256
+//   29.3 -> 22.1, 30 x 67-87 after 1915 580 -> 390.
 // Each group re-reads its keys (through L2), so long streams under many rows
 // stay with the 256-slot kernels; choose_fan (cev_host.cpp) draws the line.
 namespace fan {
@@ -1665,6 +1666,38 @@ struct Cursor {
 };
 }  // namespace fan
 
+// f32: a value as the sum of three bf16 parts (round to nearest each; exact),
+// and six of the nine part products of two such operands, small ones first
+// (the dropped three are below 2^-26).  Six 32x32x16 bf16 MFMAs take 192
+// cycles where the f32 unit takes 512 for the same 16 products; splitting the
+// keys and values costs their wave about as much again, so a sub-tile round
+// went from 5.2 to 4 us (30 x 67-87 rows after 1915 keys 443 -> 390 us).  The
+// error against f64 is smaller (5.1e-7 against 6.0e-7 there): an accumulator
+// is rounded 48 times a sub-tile instead of 64.
+namespace split {
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void parts(const float* x, bf16x8* p) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    f32x2 r = {x[e], x[e + 1]};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const bf16x2 b = __builtin_convertvector(r, bf16x2);
+      p[i][e] = b[0];
+      p[i][e + 1] = b[1];
+      r = r - __builtin_convertvector(b, f32x2);
+    }
+  }
+}
+__device__ __forceinline__ f32x16 mma(const bf16x8* a, const bf16x8* b, f32x16 c) {
+#pragma unroll
+  for (int o = 2; o >= 0; --o)
+#pragma unroll
+    for (int i = 0; i <= o; ++i) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[o - i], c, 0, 0, 0);
+  return c;
+}
+}  // namespace split
+
 template <typename T, int D>
 constexpr int kFanMinWaves = sizeof(T) == 2 && D == 128 ? 2 : 1;
 template <typename T, int D>
@@ -1706,8 +1739,27 @@ __global__ __launch_bounds__(kFanWaves * 64) __attribute__((amdgpu_waves_per_eu(
   sr.row = sr.ok ? r0 + (n >> gs) : 0;
   sr.head = kvh * a.g + (n & (a.g - 1));
 
-  F fr;
-  fr.load_q((const T*)a.q + (int64_t)sr.row * a.q_st + (int64_t)sr.head * a.q_sh, sr.ok, u);
+  const T* const qrow = (const T*)a.q + (int64_t)sr.row * a.q_st + (int64_t)sr.head * a.q_sh;
+  F fr;                         // bf16
+  bf16x8 qp[BF ? 1 : D / 16][3];  // f32: the parts of q[16 st + 8 u ..]
+  auto load_q8 = [&](int st, float* x) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) {
+      const f32x4 v = sr.ok ? *(const f32x4*)(qrow + 16 * st + 8 * u + e) : f32x4{};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[e + j] = v[j];
+    }
+  };
+  if constexpr (BF) {
+    fr.load_q(qrow, sr.ok, u);
+  } else {
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) {
+      float x[8];
+      load_q8(st, x);
+      split::parts(x, qp[st]);
+    }
+  }
   int4 rv = ((const int4*)(a.plan + ph.rows_off))[sr.row];
   if (!sr.ok) rv = make_int4(0, 0, -1, 0);
   fan::Cursor cur;
@@ -1760,7 +1812,11 @@ __global__ __launch_bounds__(kFanWaves * 64) __attribute__((amdgpu_waves_per_eu(
   auto load_k = [&](const Chunk& x, int buf) {
     kvs.rsrc(x, rk, rvs, kr, vr);
 #pragma unroll
-    for (int i = 0; i < kKLoads; ++i) kf[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, n * kr + 32 * i + 16 * u, 0, 0));
+    for (int i = 0; i < kKLoads; ++i) {
+      // bf16: 8 values at 16 i + 8 u; f32: 4 values at 16 (i / 2) + 8 u + 4 (i % 2)
+      const int at = BF ? 32 * i + 16 * u : 64 * (i >> 1) + 32 * u + 16 * (i & 1);
+      kf[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, n * kr + at, 0, 0));
+    }
     if constexpr (BF) {
       constexpr int kRows = 1024 / kRB, kBlk = kRB / 16;  // rows of one 1 KB DMA, 16-byte blocks of a row
 #pragma unroll
@@ -1785,97 +1841,149 @@ __global__ __launch_bounds__(kFanWaves * 64) __attribute__((amdgpu_waves_per_eu(
     return i < c_end && cur.seek(i, x);
   };
 
+  // f32: an infinite value (or one above bf16's range) has no parts.  A wave
+  // that ends with anything non-finite walks its keys again on the f32 unit.
+  bool exact = false;
+  const int c_first = c;
   Chunk ch, chn;
-  bool more = at(c, ch);
-  int buf = 0;
-  load_k(ch, 0);
-  load_v();
-  while (more) {
-    f32x16 s = f32x16{};
+  bool more;
+  int buf;
+  for (;;) {
+    more = at(c, ch);
+    buf = 0;
+    load_k(ch, 0);
+    load_v();
+    while (more) {
+      f32x16 s = f32x16{};
 #pragma unroll
-    for (int st = 0; st < kKLoads; ++st) {
-      if constexpr (BF) {
-        fr.qk_mfma(__builtin_bit_cast(bf16x8, kf[st]), st, s);
-      } else {
+      for (int st = 0; st < D / 16; ++st) {
+        if constexpr (BF) {
+          fr.qk_mfma(__builtin_bit_cast(bf16x8, kf[st]), st, s);
+        } else {
+          float x[8];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[st][r], fr.q[st][r], s, 0, 0, 0);
+          for (int e = 0; e < 8; ++e) x[e] = kf[2 * st + (e >> 2)][e & 3];
+          if (!exact) {
+            bf16x8 kp[3];
+            split::parts(x, kp);
+            s = split::mma(kp, qp[st], s);
+          } else {
+            float q[8];
+            load_q8(st, q);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], q[e], s, 0, 0, 0);
+          }
+        }
       }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    c += NW;
-    more = at(c, chn);
-    load_k(chn, buf ^ 1);
-    __builtin_amdgcn_sched_barrier(0);
-    if (ch.local != 0 || ch.nvalid < 32) {
-      // Branch-free on purpose (see attn_kernel_seq).
-      const bool all_rows = ch.local == 0;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int kk = 8 * (i >> 2) + 4 * u + (i & 3);
-        const int key = ch.key0 + kk;
-        const bool vis = (kk < ch.nvalid) & (all_rows | ((key >= rv.x) & (key < rv.y)) | (key == rv.z));
-        s[i] = vis ? s[i] : -INFINITY;
-      }
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    const float m_cand = pair_max(mx) * a.scale_log2;
-    const bool grow = m_cand > m_run + kRescale;
-    if (__ballot(grow)) {
-      const float m_new = grow ? m_cand : m_run;
-      const float alpha = fast_exp2(m_run - m_new);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = fast_exp2(__builtin_fmaf(s[i], a.scale_log2, -m_run));
-    P p;
-    F::make_p(s, p, l_run);
-    if constexpr (BF) {
-      // This sub-tile's V is in LDS once only the next one's loads are in
-      // flight.  The V^T reads go through asm (pipe::read_tr): the compiler
-      // would wait for the next sub-tile's DMA before each.
-      pipe::wait_vmcnt<kKLoads + kVLoads>();
-      asm volatile("" ::: "memory");
-      const int va = lds_v + buf * (32 * kRB);
-      constexpr int kGrp = 4;
-      pipe::i32x2 f[2][kGrp][2];
-      auto issue = [&](auto g_c) {
-        constexpr int G = decltype(g_c)::value;
-        static_for<kGrp>([&](auto e_c) {
-          constexpr int E = decltype(e_c)::value, J = G * kGrp + E;
-          constexpr int OFF = 16 * (J / NDT) * kRB;
-          f[G & 1][E][0] = pipe::read_tr<OFF>(va + voff[J % NDT]);
-          f[G & 1][E][1] = pipe::read_tr<OFF + 8 * kRB>(va + voff[J % NDT]);
-        });
-      };
-      issue(std::integral_constant<int, 0>{});
-      static_for<F::NPV / kGrp>([&](auto g_c) {
-        constexpr int G = decltype(g_c)::value;
-        static_for<kGrp>([&](auto e_c) {
-          constexpr int E = decltype(e_c)::value;
-          pipe::wait_tr<0>(f[G & 1][E][0], f[G & 1][E][1]);
-        });
-        if constexpr (G + 1 < F::NPV / kGrp) issue(std::integral_constant<int, G + 1>{});
-        static_for<kGrp>([&](auto e_c) {
-          constexpr int E = decltype(e_c)::value;
-          const bf16x4 lo = __builtin_bit_cast(bf16x4, f[G & 1][E][0]), hi = __builtin_bit_cast(bf16x4, f[G & 1][E][1]);
-          F::pv_mfma(bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, G * kGrp + E, p, o);
-        });
-      });
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[i][dt], p.v[i], o[dt], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      load_v();
+      c += NW;
+      more = at(c, chn);
+      load_k(chn, buf ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (ch.local != 0 || ch.nvalid < 32) {
+        // Branch-free on purpose (see attn_kernel_seq).
+        const bool all_rows = ch.local == 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int kk = 8 * (i >> 2) + 4 * u + (i & 3);
+          const int key = ch.key0 + kk;
+          const bool vis = (kk < ch.nvalid) & (all_rows | ((key >= rv.x) & (key < rv.y)) | (key == rv.z));
+          s[i] = vis ? s[i] : -INFINITY;
+        }
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
+      const float m_cand = pair_max(mx) * a.scale_log2;
+      const bool grow = m_cand > m_run + kRescale;
+      if (__ballot(grow)) {
+        const float m_new = grow ? m_cand : m_run;
+        const float alpha = fast_exp2(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = fast_exp2(__builtin_fmaf(s[i], a.scale_log2, -m_run));
+      P p;
+      F::make_p(s, p, l_run);
+      if constexpr (BF) {
+        // This sub-tile's V is in LDS once only the next one's loads are in
+        // flight.  The V^T reads go through asm (pipe::read_tr): the compiler
+        // would wait for the next sub-tile's DMA before each.
+        pipe::wait_vmcnt<kKLoads + kVLoads>();
+        asm volatile("" ::: "memory");
+        const int va = lds_v + buf * (32 * kRB);
+        constexpr int kGrp = 4;
+        pipe::i32x2 f[2][kGrp][2];
+        auto issue = [&](auto g_c) {
+          constexpr int G = decltype(g_c)::value;
+          static_for<kGrp>([&](auto e_c) {
+            constexpr int E = decltype(e_c)::value, J = G * kGrp + E;
+            constexpr int OFF = 16 * (J / NDT) * kRB;
+            f[G & 1][E][0] = pipe::read_tr<OFF>(va + voff[J % NDT]);
+            f[G & 1][E][1] = pipe::read_tr<OFF + 8 * kRB>(va + voff[J % NDT]);
+          });
+        };
+        issue(std::integral_constant<int, 0>{});
+        static_for<F::NPV / kGrp>([&](auto g_c) {
+          constexpr int G = decltype(g_c)::value;
+          static_for<kGrp>([&](auto e_c) {
+            constexpr int E = decltype(e_c)::value;
+            pipe::wait_tr<0>(f[G & 1][E][0], f[G & 1][E][1]);
+          });
+          if constexpr (G + 1 < F::NPV / kGrp) issue(std::integral_constant<int, G + 1>{});
+          static_for<kGrp>([&](auto e_c) {
+            constexpr int E = decltype(e_c)::value;
+            const bf16x4 lo = __builtin_bit_cast(bf16x4, f[G & 1][E][0]), hi = __builtin_bit_cast(bf16x4, f[G & 1][E][1]);
+            F::pv_mfma(bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, G * kGrp + E, p, o);
+          });
+        });
+      } else {
+        if (!exact) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = p.v[8 * h + e];
+            bf16x8 pp[3];
+            split::parts(x, pp);
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) x[e] = vf[8 * h + e][dt];
+              bf16x8 vp[3];
+              split::parts(x, vp);
+              o[dt] = split::mma(vp, pp, o[dt]);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[i][dt], p.v[i], o[dt], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_v();
+      }
+      ch = chn;
+      buf ^= 1;
     }
-    ch = chn;
-    buf ^= 1;
+    if constexpr (BF) break;
+    float t = l_run * 0.0f + m_run * 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t += o[dt][i] * 0.0f;
+    if (exact || !__any(!(t == 0.0f))) break;
+    exact = true;
+    c = c_first;
+    cur.start();
+    m_run = -1e30f;
+    l_run = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
   }
   // loads past the end still write zeros into LDS: drain them
   if (BF) pipe::wait_vmcnt<0>();

@@ -381,6 +381,29 @@ def test_small_launches_vs_oracle(gpu, orc, dtype, hq, hkv, d, gated, case):
         assert_f32(got, want, f"{case} d={d}")
 
 
+def test_small_f32_launch_keeps_infinities(gpu):
+    """Infinite keys and values have no bf16 parts: the waves that meet them
+    walk their keys again on the f32 unit.  Where the 256-slot kernel gives an
+    infinity this one gives the same, and where it is finite so is this one
+    (a masked infinite value is 0 * inf for every row it is loaded with, which
+    here are fewer rows)."""
+    import torch
+    tab, _, _ = cev_hip.BlockTable.from_plans([(47, 47, 47)], [(0, 40), (0, 33), (0, 35)])
+    t, s, hq, hkv, d = tab.t, tab.s_cache, 16, 8, 128
+    g = torch.Generator().manual_seed(9)
+    rnd = lambda *sh: torch.randn(*sh, generator=g).to(gpu)  # noqa: E731
+    q, kn, vn, kc, vc = rnd(t, hq, d), rnd(t, hkv, d), rnd(t, hkv, d), rnd(hkv, s, d), rnd(hkv, s, d)
+    vn[45, 2, 7], kn[80, 3, 9] = float("inf"), float("inf")
+    op = cev_hip.PackedAttention(q, kn, tab, k_cache=kc, s_cache=s, v_new=vn, v_cache=vc)
+    assert int(op.plan.header()[18]) == 1
+    got = op(q, kn, vn, kc, vc)
+    want = cev_hip.packed_attention(q, kn, vn, tab, k_cache=kc, v_cache=vc, max_splits=1)
+    fin = torch.isfinite(want)
+    inf = torch.isinf(want)
+    assert inf.any() and torch.equal(got[inf], want[inf])
+    assert (got[fin] - want[fin]).abs().max() <= F32_TOL
+
+
 def test_packed_equals_each_block_alone_on_gpu(gpu):
     """qwen3.rs:13-17: packing is exactly asking each question alone.  The
     kernel visits the same key tiles in the same order either way (unsplit),
