@@ -327,7 +327,12 @@ void choose_fan(const cev_attn_desc* d, Plan& p) {
     if (!bf)
       us += 3.0 + std::max(8.0 + 4.0 * r, cu_rounds * (8.0 + 4.0 * avg));
     else if (wide)
-      us += 3.0 + std::max(10.0 + 2.0 * r, cu_rounds * (10.0 + 2.0 * avg));
+      // more than one CU round: the CUs share the L2's bandwidth, and the
+      // longest groups do not start first.  480 workgroups of at most 4
+      // sub-tile rounds took 41-50 us where 10 + 2 avg a CU round said 31-38
+      // (the whole call, 9 x 68-86 rows after 126 + 288 keys: 62 us, in
+      // 256-slot form 57)
+      us += 3.0 + (cu_rounds > 1.0 ? cu_rounds * (7.5 + 2.0 * (avg + r)) : 10.0 + 2.0 * r);
     else
       us += 6.0 + std::max(1.2 * r, cu_rounds * (1.25 * avg + 1.6));
     if (us < best) {
