@@ -1,5 +1,5 @@
 // Attention plan blob shared by the host planner (cev_host.cpp) and the
-// packed-attention launcher / kernel (packed_attn.hip).
+// packed-attention launcher and kernels (packed_attn.hip, fan_attn.hip).
 //
 // Layout (all int32, 16-byte aligned sections):
 //   header                 16 x int32

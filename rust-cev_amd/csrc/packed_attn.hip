@@ -26,533 +26,10 @@
 //     workspace and attn_merge_kernel combines the parts.
 #include <atomic>
 #include <mutex>
-#include <type_traits>
 
-#include "cev_device.h"
-#include "cev_internal.h"
-#include "cev_plan.h"
+#include "attn_device.h"
 
 namespace {
-
-struct AttnArgs {
-  const void* q;
-  const void* kc;
-  const void* vc;
-  const void* kn;
-  const void* vn;
-  const void* gate;
-  void* out;
-  char* ws;  // split records: outputs, then (m, l) pairs (cev_plan.h)
-  const int32_t* plan;
-  int64_t q_st, q_sh, kc_ss, kc_sh, vc_ss, vc_sh, kn_st, kn_sh, vn_st, vn_sh, g_st, g_sh, o_st, o_sh;
-  int32_t n_tiles, t, s_cache, hq, hkv, g, has_gate, n_splits, tile_rows;
-  int32_t fan_parts, fan_subs;  // attn_kernel_fan: parts of the key stream (0: not this form), 32-slot groups per tile
-  int32_t rows_dense;  // the host plan's tiles cover rows [0, t) in order, each row once
-  float scale_log2;
-  uint32_t plan_sig;  // signature of the host plan this launch was validated with
-};
-
-constexpr float kRescale = 8.0f;
-// Largest sum of a lane's 16 probabilities of one sub-tile that the d = 128
-// loop accepts before it moves the row's max (so p < 2^16 there).
-constexpr float kMaxP = 65536.0f;
-constexpr float kLog2MaxP = 16.0f;  // log2(kMaxP)
-
-// The plan header on the device must be the host plan's (same signature,
-// same launch shape).  A device plan that is not a copy of the validated
-// host plan is never followed: the attention kernels fill the whole output
-// with NaN instead (poison_output) and the merge pass writes nothing, so a
-// stale device plan shows in the result rather than leaving rows unwritten.
-// The header is read at once and every field compared (no short-circuit,
-// which would make each field a dependent load).
-// The header stays in h for the offsets the kernel reads next.
-__device__ __forceinline__ bool header_ok(const AttnArgs& a, const cev_plan_header& h) {
-  // the section offsets follow the header in order (this also loads them
-  // with the other fields)
-  constexpr int32_t kHeaderWords = (int32_t)(sizeof(cev_plan_header) / 4);
-  return (h.magic == CEV_PLAN_MAGIC) & ((uint32_t)h.sig == a.plan_sig) & (h.n_tiles == a.n_tiles) & (h.t == a.t) &
-         (h.s_cache == a.s_cache) & (h.n_splits == a.n_splits) & (h.tiles_off >= kHeaderWords) & (h.segs_off >= h.tiles_off) &
-         (h.rows_off >= h.segs_off);
-}
-__device__ __forceinline__ bool plan_ok(const AttnArgs& a, cev_plan_header& h) {
-  h = *(const cev_plan_header*)a.plan;
-  return header_ok(a, h);
-}
-
-// Workgroup b of the grid writes NaN over output rows [b t / G, (b+1) t / G)
-// of every query head (the launcher validated the output strides).
-template <typename T, int D>
-__device__ void poison_output(const AttnArgs& a) {
-  const int64_t G = gridDim.x;
-  const int64_t r0 = (int64_t)blockIdx.x * a.t / G, r1 = (int64_t)(blockIdx.x + 1) * a.t / G;
-  const int64_t per_row = (int64_t)a.hq * D;
-  for (int64_t i = threadIdx.x; i < (r1 - r0) * per_row; i += blockDim.x) {
-    const int64_t r = r0 + i / per_row, h = (i % per_row) / D, e = i % D;
-    ((T*)a.out)[r * a.o_st + h * a.o_sh + e] = (T)__builtin_nanf("");
-  }
-}
-
-// Clamps a segment to the key buffer it starts in.
-__device__ __forceinline__ int4 clamp_seg(int4 sg, int s_cache, int t) {
-  sg.x = max(sg.x, 0);
-  const int lim = sg.x < s_cache ? s_cache : s_cache + t;
-  sg.y = min(sg.y, lim);
-  return sg;
-}
-
-__device__ __forceinline__ float gate_value(float o, float g, bool bf16) {
-  // out * sigmoid(g), each op in the model dtype (qwen35.rs:556-558)
-  if (bf16) {
-    float e = bf16_round(expf(-g));
-    float den = bf16_round(e + 1.0f);
-    // bf16(1 / den) from the hardware reciprocal (1 ulp): den = D 2^p with
-    // D an 8-bit integer, a bf16 rounding midpoint is M 2^q with M an odd
-    // 9-bit integer, and D M is never a power of two, so 1 / den lies at
-    // least 2^-17 (relative) from every midpoint and a 2^-23 error cannot
-    // change its bf16 rounding.  Below 2^-126 (den > 2^126) the reciprocal
-    // is an f32 denormal, which the division still gives exactly.
-    float sg = bf16_round(den < 0x1p126f ? __builtin_amdgcn_rcpf(den) : 1.0f / den);
-    return bf16_round(bf16_round(o) * sg);
-  }
-  return o * (1.0f / (expf(-g) + 1.0f));
-}
-
-__device__ __forceinline__ float pair_max(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-__device__ __forceinline__ float pair_sum(float x) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// The larger of x and its value in lane ^ 16 (within each 32-lane half).
-__device__ __forceinline__ float pair16_max(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-
-// x plus its value in lane ^ 16 (within each 32-lane half).
-__device__ __forceinline__ float pair16_sum(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ bf16x4 lds_read_tr(const __bf16* p) {
-  s16x4 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
-  return __builtin_bit_cast(bf16x4, r);
-}
-
-// --------------------------------------------------------------------------
-// Per-dtype MFMA fragments.
-//
-// bf16 (v_mfma_f32_32x32x16_bf16): Q as the B operand, 8 head-dim values per
-// lane per step; P converted to bf16 B operands whose K slot 8u + j of half
-// h is S^T register 8h + j (key 16h + 8(j/4) + 4u + j%4 of a sub-tile); the
-// V^T A operand comes from ds_read_b64_tr_b16 on the key-major V tile.
-//
-// f32 (v_mfma_f32_32x32x2_f32, full f32 products): the head-dim order of
-// the QK^T K slots is permuted (d = 8k + 4u + r) so a lane reads 4
-// consecutive floats for 4 steps; one K=2 PV step per S^T register.
-//
-// Both expose the work as small steps so the main loop can interleave the
-// MFMAs of one sub-tile with the VALU work of another:
-//   qk_step(st), st < NQK   - builds one 32x32 S^T sub-tile;
-//   pv_step(j),  j < NPV    - adds one sub-tile's V^T . P^T to O;
-//   make_p                  - probabilities -> PV operand, plus their sum.
-template <typename T, int D>
-struct Frag;
-
-#ifndef CEV_VPAD_BF16
-#define CEV_VPAD_BF16 32
-#endif
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-template <int D>
-struct Frag<__bf16, D> {
-  static constexpr int BN = D == 128 ? 64 : 32;
-  static constexpr int PAD = 8;
-  static constexpr int VPAD = CEV_VPAD_BF16;
-  static constexpr int VEC = 8;
-  static constexpr int NQK = D / 16;
-  static constexpr int NPV = 2 * (D / 32);
-  typedef bf16x8 Vec;
-  struct P {
-    bf16x8 h[2];
-  };
-  bf16x8 q[D / 16];
-
-  __device__ __forceinline__ void load_q(const __bf16* qp, bool ok, int u) {
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) {
-      bf16x8 z = {};
-      q[s] = ok ? *(const bf16x8*)(qp + 16 * s + 8 * u) : z;
-    }
-  }
-  // q * c rounded to bf16: the QK^T MFMAs then give scores already in the
-  // base-2 units of the softmax (c = scale * log2 e).
-  __device__ __forceinline__ void scale_q(float c) {
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) q[s][e] = (__bf16)((float)q[s][e] * c);
-  }
-
-  // K operand of QK step st: key kt*32 + n, head-dim values 16st + 8u ..
-  template <int RS>
-  __device__ __forceinline__ static bf16x8 k_frag(const __bf16* sK, int kt, int st, int n, int u) {
-    return *(const bf16x8*)&sK[(kt * 32 + n) * RS + 16 * st + 8 * u];
-  }
-  __device__ __forceinline__ void qk_mfma(const bf16x8& af, int st, f32x16& s) const {
-    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, q[st], s, 0, 0, 0);
-  }
-  template <int RS>
-  __device__ __forceinline__ void qk_step(const __bf16* sK, int kt, int st, int n, int u, f32x16& s) const {
-    qk_mfma(k_frag<RS>(sK, kt, st, n, u), st, s);
-  }
-
-  // The row sum is taken over the bf16 probabilities PV multiplies, on the
-  // dot-product unit (two products per instruction).
-  __device__ __forceinline__ static void make_p(const f32x16& e, P& p, float& rs) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p.h[h][j] = (__bf16)e[8 * h + j];
-    const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) rs = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{p.h[h][j], p.h[h][j + 1]}, one, rs, false);
-  }
-
-  // Step j = h * (D/32) + dt: o[dt] += V^T(keys of half h) . P^T(half h).
-  // Lane (group g16 = lane/16, i = lane%16) reads row kb + i/4, columns
-  // d0 + 4(i%4) .. +3; the transpose load hands it 4 consecutive keys of
-  // head-dim column d0 + i.
-  template <int RS>
-  __device__ __forceinline__ static bf16x8 v_frag(const __bf16* sV, int kt, int j, int lane, int u) {
-    const int h = j / (D / 32), dt = j % (D / 32);
-    const int tr_row = (lane & 15) >> 2;
-    const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-    const __bf16* vp = sV + (kt * 32 + 16 * h + 4 * u + tr_row) * RS + dt * 32 + tr_col;
-    const bf16x4 lo = lds_read_tr(vp);
-    const bf16x4 hi = lds_read_tr(vp + 8 * RS);
-    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-  }
-  __device__ __forceinline__ static void pv_mfma(const bf16x8& af, int j, const P& p, f32x16* o) {
-    const int h = j / (D / 32), dt = j % (D / 32);
-    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, p.h[h], o[dt], 0, 0, 0);
-  }
-  template <int RS>
-  __device__ __forceinline__ void pv_step(const __bf16* sV, int kt, int j, int lane, int u, const P& p, f32x16* o) const {
-    pv_mfma(v_frag<RS>(sV, kt, j, lane, u), j, p, o);
-  }
-};
-
-template <int D>
-struct Frag<float, D> {
-  static constexpr int BN = 32;
-  static constexpr int PAD = 4;
-  static constexpr int VPAD = 4;
-  static constexpr int VEC = 4;
-  static constexpr int NQK = D / 8;
-  static constexpr int NPV = 16;
-  typedef f32x4 Vec;
-  struct P {
-    f32x16 v;
-  };
-  f32x4 q[D / 8];
-
-  __device__ __forceinline__ void load_q(const float* qp, bool ok, int u) {
-#pragma unroll
-    for (int k = 0; k < D / 8; ++k) q[k] = ok ? *(const f32x4*)(qp + 8 * k + 4 * u) : f32x4{};
-  }
-
-  template <int RS>
-  __device__ __forceinline__ void qk_step(const float* sK, int kt, int k, int n, int u, f32x16& s) const {
-    const f32x4 af = *(const f32x4*)&sK[(kt * 32 + n) * RS + 8 * k + 4 * u];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) s = __builtin_amdgcn_mfma_f32_32x32x2f32(af[r], q[k][r], s, 0, 0, 0);
-  }
-
-  __device__ __forceinline__ static void make_p(const f32x16& e, P& p, float& rs) {
-    p.v = e;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) rs += e[i];
-  }
-
-  template <int RS>
-  __device__ __forceinline__ void pv_step(const float* sV, int kt, int i, int lane, int u, const P& p, f32x16* o) const {
-    const int n = lane & 31;
-    const int key = kt * 32 + 8 * (i >> 2) + 4 * u + (i & 3);
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(sV[key * RS + dt * 32 + n], p.v[i], o[dt], 0, 0, 0);
-  }
-};
-
-template <typename T>
-__device__ __forceinline__ void store_vec4(T* p, const float* v);
-template <>
-__device__ __forceinline__ void store_vec4<__bf16>(__bf16* p, const float* v) {
-  bf16x4 r = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-  *(bf16x4*)p = r;
-}
-template <>
-__device__ __forceinline__ void store_vec4<float>(float* p, const float* v) {
-  *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]};
-}
-
-template <typename T>
-__device__ __forceinline__ void load_vec4(const T* p, float* v);
-template <>
-__device__ __forceinline__ void load_vec4<__bf16>(const __bf16* p, float* v) {
-  const bf16x4 g = *(const bf16x4*)p;
-  for (int e = 0; e < 4; ++e) v[e] = (float)g[e];
-}
-template <>
-__device__ __forceinline__ void load_vec4<float>(const float* p, float* v) {
-  const f32x4 g = *(const f32x4*)p;
-  for (int e = 0; e < 4; ++e) v[e] = g[e];
-}
-
-// Four values of a record's output as loaded (bf16x4 or f32x4) and their
-// f32 form.
-template <typename T>
-using VecOf = typename std::conditional<sizeof(T) == 2, bf16x4, f32x4>::type;
-// E values of T as one load or store: bf16x8 for E = 8, else VecOf<T>.
-template <typename T, int E>
-using VecN = typename std::conditional<E == 8, bf16x8, VecOf<T>>::type;
-__device__ __forceinline__ f32x4 to_f32x4(const bf16x4& v) { return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}; }
-__device__ __forceinline__ f32x4 to_f32x4(const f32x4& v) { return v; }
-
-// The normalised, optionally gated output of one query slot (row, head):
-// lane half ue holds columns 32 dt + 8 q4 + 4 ue .. +3 of o[dt].  bf16
-// layers multiply by 1/l (the result is rounded to bf16), f32 layers divide
-// by l.  The gate's loads are all issued before the first store, so each of
-// the row's output lines is written in one burst; with one load round trip
-// between stores, lines sat half written in L2 and went to HBM twice.
-template <typename T, int D>
-__device__ __forceinline__ void store_output(const AttnArgs& a, int row, int head, int ue, const f32x16* o, float l) {
-  constexpr int NDT = D / 32;
-  constexpr bool BF = sizeof(T) == 2;
-  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  T* op = (T*)a.out + (int64_t)row * a.o_st + (int64_t)head * a.o_sh;
-  auto value = [&](int dt, int i) { return BF ? o[dt][i] * inv : (l > 0.0f ? o[dt][i] / l : 0.0f); };
-  if (a.has_gate) {
-    const T* gp = (const T*)a.gate + (int64_t)row * a.g_st + (int64_t)head * a.g_sh;
-    VecOf<T> graw[NDT][4];
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) graw[dt][q4] = *(const VecOf<T>*)(gp + dt * 32 + 8 * q4 + 4 * ue);
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const f32x4 gv = to_f32x4(graw[dt][q4]);
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = gate_value(value(dt, 4 * q4 + e), gv[e], BF);
-        store_vec4<T>(op + dt * 32 + 8 * q4 + 4 * ue, v);
-      }
-  } else {
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = value(dt, 4 * q4 + e);
-        store_vec4<T>(op + dt * 32 + 8 * q4 + 4 * ue, v);
-      }
-  }
-}
-
-// Index of record (row, head, part) in the split workspace.
-__device__ __forceinline__ int64_t record_index(const AttnArgs& a, int row, int head, int part) {
-  return ((int64_t)row * a.hq + head) * a.n_splits + part;
-}
-// Output of record i, and the (m, l) region that follows all outputs.
-template <typename T, int D>
-__device__ __forceinline__ T* record_out(const AttnArgs& a, int64_t i) {
-  return (T*)a.ws + i * D;
-}
-template <typename T, int D>
-__device__ __forceinline__ float2* record_ml(const AttnArgs& a) {
-  return (float2*)(a.ws + (int64_t)a.t * a.hq * a.n_splits * D * (int64_t)sizeof(T));
-}
-
-// Writes this lane's share of partial record (row, head, part): output
-// values d .. d+3 of every (dt, q4) slice (d = 32 dt + 8 q4 + 4u), then m
-// and l from the lane with u == 0.
-template <typename T, int D>
-__device__ __forceinline__ void write_record(const AttnArgs& a, int row, int head, int part, const f32x16* o, int u, float m, float l) {
-  const int64_t i = record_index(a, row, head, part);
-  T* rec = record_out<T, D>(a, i);
-#pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4) {
-      const int d = dt * 32 + 8 * q4 + 4 * u;
-      const float v[4] = {o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
-      store_vec4<T>(rec + d, v);
-    }
-  if (u == 0) record_ml<T, D>(a)[i] = make_float2(m, l);
-}
-
-// Word 3 of a raw buffer resource on gfx9: 32-bit data format, no swizzle.
-constexpr int kBufferWord3 = 0x00020000;
-
-// Values the compiler cannot prove wave-uniform (they come through vector
-// loads of the plan) but are: readfirstlane moves them to SGPRs, where a
-// buffer resource must live.
-__device__ __forceinline__ int uniform_i32(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
-
-// Keeps a value computed where it stands: sched_barrier only fences the
-// machine scheduler, and without a use the IR passes sink the row max and
-// row sum past the MFMAs they are meant to overlap.
-__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
-
-// One BN-key chunk of a tile's key stream: keys key0 .. key0 + BN, the first
-// nvalid of them inside the segment; local != 0 when the segment's keys are
-// masked per row.
-struct Chunk {
-  int key0, nvalid, local;
-};
-
-// Cursor over the BN-key chunks of a tile's segments.  The current segment,
-// clamped, stays in SGPRs; the plan is read only when the cursor enters a
-// new segment (readfirstlane tells the compiler these vector-loaded values
-// are wave-uniform).
-template <int BN>
-struct ChunkCursor {
-  const int4* segs;
-  int nseg, s_cache, t;
-  int si, k0;
-  int4 cur;
-
-  __device__ __forceinline__ int4 seg(int i) const {
-    const int4 sg = clamp_seg(segs[i], s_cache, t);
-    return make_int4(uniform_i32(sg.x), uniform_i32(sg.y), uniform_i32(sg.z), 0);
-  }
-  // Positions the cursor on chunk c of the tile's stream.
-  __device__ __forceinline__ void seek(int c) {
-    si = 0;
-    k0 = 0;
-    cur = make_int4(0, 0, 0, 0);
-    for (; si < nseg; ++si) {
-      cur = seg(si);
-      const int nch = (max(0, cur.y - cur.x) + BN - 1) / BN;
-      if (c < nch) {
-        k0 = c * BN;
-        return;
-      }
-      c -= nch;
-    }
-  }
-  __device__ __forceinline__ bool valid() const { return si < nseg; }
-  __device__ __forceinline__ void next() {
-    k0 += BN;
-    if (cur.x + k0 < cur.y) return;
-    k0 = 0;
-    for (++si; si < nseg; ++si) {
-      cur = seg(si);
-      if (cur.y > cur.x) return;
-    }
-  }
-  __device__ __forceinline__ Chunk here() const {
-    Chunk ch{0, 0, 0};
-    if (si < nseg) {
-      ch.key0 = cur.x + k0;
-      ch.nvalid = max(0, min(BN, cur.y - ch.key0));
-      ch.local = cur.z;
-    }
-    return ch;
-  }
-};
-
-// K/V rows of one KV head (cache rows [0, s_cache), then the new rows),
-// fetched with buffer loads whose byte range ends at a chunk's last valid
-// key: rows past it read as zero.
-template <typename T>
-struct KvSource {
-  uint64_t kc, vc, kn, vn;         // row 0 of this head
-  int kc_rb, vc_rb, kn_rb, vn_rb;  // row strides in bytes
-  int s_cache;
-
-  __device__ __forceinline__ void init(const AttnArgs& a, int kvh) {
-    kc = (uint64_t)((const T*)a.kc + kvh * a.kc_sh);
-    vc = (uint64_t)((const T*)a.vc + kvh * a.vc_sh);
-    kn = (uint64_t)((const T*)a.kn + kvh * a.kn_sh);
-    vn = (uint64_t)((const T*)a.vn + kvh * a.vn_sh);
-    kc_rb = (int)(a.kc_ss * (int64_t)sizeof(T));
-    vc_rb = (int)(a.vc_ss * (int64_t)sizeof(T));
-    kn_rb = (int)(a.kn_st * (int64_t)sizeof(T));
-    vn_rb = (int)(a.vn_st * (int64_t)sizeof(T));
-    s_cache = a.s_cache;
-  }
-  // Buffer resources for chunk ch and the row strides they use.
-  __device__ __forceinline__ void rsrc(const Chunk& ch, __amdgpu_buffer_rsrc_t& rk, __amdgpu_buffer_rsrc_t& rv, int& kr, int& vr) const {
-    const bool cached = ch.key0 < s_cache;
-    kr = uniform_i32(cached ? kc_rb : kn_rb);
-    vr = uniform_i32(cached ? vc_rb : vn_rb);
-    const int64_t row0 = cached ? ch.key0 : ch.key0 - s_cache;
-    const uint64_t kp = uniform_u64((cached ? kc : kn) + (uint64_t)(row0 * kr));
-    const uint64_t vp = uniform_u64((cached ? vc : vn) + (uint64_t)(row0 * vr));
-    rk = __builtin_amdgcn_make_buffer_rsrc((void*)kp, (short)0, uniform_i32(ch.nvalid * kr), kBufferWord3);
-    rv = __builtin_amdgcn_make_buffer_rsrc((void*)vp, (short)0, uniform_i32(ch.nvalid * vr), kBufferWord3);
-  }
-};
-
-// Loads this thread's share of chunk ch (NLD 16-byte vectors per tensor).
-template <typename T, int D, int NLD, int NT, typename Vec>
-__device__ __forceinline__ void load_chunk(const KvSource<T>& src, const Chunk& ch, int tid, Vec* kreg, Vec* vreg) {
-  constexpr int VEC = 16 / sizeof(T);
-  __amdgpu_buffer_rsrc_t rk, rv;
-  int kr, vr;
-  src.rsrc(ch, rk, rv, kr, vr);
-#pragma unroll
-  for (int r = 0; r < NLD; ++r) {
-    const int v = tid + r * NT;
-    const int key = v / (D / VEC), col = (v % (D / VEC)) * VEC;
-    kreg[r] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b128(rk, key * kr + col * (int)sizeof(T), 0, 0));
-    vreg[r] = __builtin_bit_cast(Vec, __builtin_amdgcn_raw_buffer_load_b128(rv, key * vr + col * (int)sizeof(T), 0, 0));
-  }
-}
-
-// Query slot (wave, n = lane % 32) of a workgroup over tile rows [r0, r0 +
-// len) and KV head kvh holds tile row slot / g and query head slot % g: the
-// valid rows of a short tile fill the first waves.
-struct SlotRow {
-  int row, head, u;
-  bool ok;
-};
-__device__ __forceinline__ SlotRow slot_row(int lane, int wave, int kvh, int g, int r0, int len, int t) {
-  const int slot = wave * 32 + (lane & 31);
-  const int rit = slot / g;
-  SlotRow sr;
-  sr.ok = rit < len && r0 + rit < t;
-  sr.row = sr.ok ? r0 + rit : 0;
-  sr.head = kvh * g + slot % g;
-  sr.u = lane >> 5;
-  return sr;
-}
-
-// This lane's id, computed afresh (opaque to common-subexpression elimination).
-__device__ __forceinline__ int fresh_lane_id() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
-}
 
 // --------------------------------------------------------------------------
 // bf16, d = 128: the MFMA and VALU halves of consecutive 32-key sub-tiles
@@ -577,36 +54,13 @@ constexpr int kTileBytes = 64 * kRowBytes;
 constexpr int kVBase = kBuf * kTileBytes;  // K tiles first, then V tiles
 
 __device__ __forceinline__ int k_slot(int blk, int row) { return blk ^ (row & 15); }
-__device__ __forceinline__ int v_slot(int blk, int row) { return blk ^ ((row & 3) << 2); }
 
 // Workgroup barrier after this wave's LDS operations have completed; global
 // loads may still be in flight.  The asm is a compiler memory barrier too.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// s_waitcnt vmcnt(N) with the other counters left alone (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-// V^T operand reads.  The compiler places an s_waitcnt vmcnt(0) before
-// every ds_read_b64_tr_b16 it emits while an LDS DMA is in flight (it
-// cannot tell the buffers apart), which would drain the whole fetch
-// pipeline once per sub-tile.  These reads are issued from asm instead;
-// buffer reuse is ordered by the explicit vmcnt wait and barrier at the end
-// of each iteration, and wait_tr() below makes a fragment's registers
-// depend on the reads having returned.
-template <int OFF>
-__device__ __forceinline__ i32x2 read_tr(int vaddr) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds offset field");
-  i32x2 r;
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(vaddr), "i"(OFF) : "memory");
-  return r;
-}
 // The K operand reads go through asm as well, so that every LDS read in the
 // loop body is one whose position the waits below can count.
 template <int OFF>
@@ -619,14 +73,6 @@ __device__ __forceinline__ i32x4 read_b128(int vaddr) {
 // One K operand fragment: a 16-byte read per lane.  Two 8-byte reads of
 // the same bytes measured no faster; the reads are bound by LDS bytes.
 typedef i32x4 KFrag;
-// LDS returns in order: once at most N LGKM operations are outstanding,
-// every LDS read issued before the last N LDS reads has landed (an older
-// scalar load still in flight only makes the wait stricter).
-template <int N>
-__device__ __forceinline__ void wait_tr(i32x2& lo, i32x2& hi) {
-  static_assert(N >= 0 && N < 16, "lgkmcnt range");
-  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(lo), "+v"(hi) : "i"(N));
-}
 template <int N>
 __device__ __forceinline__ void wait_b128(i32x4& r) {
   static_assert(N >= 0 && N < 16, "lgkmcnt range");
@@ -1571,489 +1017,6 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_kernel_wide(AttnArgs a) 
   store_output<T, D>(a, sr.row, sr.head, ue, o, l);
 }
 
-// --------------------------------------------------------------------------
-// Small launches, every dtype and head dim: a workgroup of kFanWaves waves
-// holds 32 query slots and its waves take the 32-key sub-tiles of the key
-// stream in turn, then combine their partials through LDS.
-//
-// The kernels above give a workgroup 256 slots.  With few query rows that
-// leaves most CUs idle while one CU's four SIMDs issue the softmax, mask and
-// (gated) epilogue instructions of all 256 slots, each instruction 4 cycles
-// a wave: an 8-workgroup launch measured 15 us and a gated d = 256 one 40 us
-// with 2 us of MFMA work.  Here a launch has eight times the workgroups, a
-// group's masked keys are cut to the ones its own rows see, and a wave
-// carries one sub-tile's worth of every phase.  No barrier until the
-// combine: K goes to registers, V into this wave's own LDS (bf16, by DMA
-// and read back transposed) or registers (f32), one sub-tile ahead.
-// K2 with its merge, traced, before -> now:
-//   bf16 d = 128: 1 x 19 tokens after 301 keys 15.0 -> 9.5 us, 8 x 61-77
-//   after 74 25.5 -> 11.6, 11 x 21-44 after 421 31.4 -> 16.6;
-//   bf16 d = 256 gated: 5 rows of 43 40.0 -> 14.7, 4 x 28-40 after 123
-//   42.6 -> 16.2;  f32: 5 x 33-43 after 47 31.2 -> 14.2, 12 x 32 after 256
-//   29.3 -> 22.1, 30 x 67-87 after 1915 580 -> 390.
-// Each group re-reads its keys (through L2), so long streams under many rows
-// stay with the 256-slot kernels; choose_fan (cev_host.cpp) draws the line.
-namespace fan {
-// The smallest x of the 32 lanes of a wave half.
-__device__ __forceinline__ int half_min(int x) {
-  x = min(x, (int)dpp_u<0xB1>((uint32_t)x));
-  x = min(x, (int)dpp_u<0x4E>((uint32_t)x));
-  x = min(x, (int)dpp_u<0x141>((uint32_t)x));
-  x = min(x, (int)dpp_u<0x140>((uint32_t)x));
-  auto r = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
-  return min((int)r[0], (int)r[1]);
-}
-
-// Cursor over the 32-key sub-tiles of a tile's segments.  Lane l keeps
-// segment 64 b + l of the current batch b of 64, with masked segments cut to
-// the keys [lo, hi) that some row of this workgroup's slots can see.
-struct Cursor {
-  const int4* segs;
-  int nseg, s_cache, t, lo, hi;
-  int4 batch;
-  int si, c_base, nch;
-  Chunk seg;  // key0 = first key of segment si, nvalid = its keys
-
-  __device__ __forceinline__ void load_batch(int b) {
-    const int i = min(64 * b + (int)(threadIdx.x & 63), nseg - 1);
-    int4 sg = clamp_seg(segs[i], s_cache, t);
-    if (sg.z) {
-      sg.x = max(sg.x, lo);
-      sg.y = min(sg.y, hi);
-    }
-    sg.y = max(sg.y, sg.x);
-    batch = sg;
-  }
-  __device__ __forceinline__ void enter() {
-    if (si >= nseg) return;
-    if (si > 0 && (si & 63) == 0) load_batch(si >> 6);
-    const int l = si & 63;
-    seg.key0 = __builtin_amdgcn_readlane(batch.x, l);
-    seg.nvalid = __builtin_amdgcn_readlane(batch.y, l) - seg.key0;
-    seg.local = __builtin_amdgcn_readlane(batch.z, l);
-    nch = (seg.nvalid + 31) >> 5;
-  }
-  __device__ __forceinline__ void start() {
-    si = 0;
-    c_base = 0;
-    nch = 0;
-    seg = Chunk{0, 0, 0};
-    if (nseg > 0) load_batch(0);
-    enter();
-  }
-  // Sub-tile c (never before the current segment); false past the end.
-  __device__ __forceinline__ bool seek(int c, Chunk& ch) {
-    while (si < nseg && c >= c_base + nch) {
-      c_base += nch;
-      ++si;
-      enter();
-    }
-    if (si >= nseg) return false;
-    const int k0 = 32 * (c - c_base);
-    ch.key0 = seg.key0 + k0;
-    ch.nvalid = min(32, seg.nvalid - k0);
-    ch.local = seg.local;
-    return true;
-  }
-  __device__ __forceinline__ int total() {
-    while (si < nseg) {
-      c_base += nch;
-      ++si;
-      enter();
-    }
-    return c_base;
-  }
-};
-}  // namespace fan
-
-// f32: a value as the sum of three bf16 parts (round to nearest each; exact),
-// and six of the nine part products of two such operands, small ones first
-// (the dropped three are below 2^-26).  Six 32x32x16 bf16 MFMAs take 192
-// cycles where the f32 unit takes 512 for the same 16 products; splitting the
-// keys and values costs their wave about as much again, so a sub-tile round
-// went from 5.2 to 4 us (30 x 67-87 rows after 1915 keys 443 -> 390 us).  The
-// error against f64 is smaller (5.1e-7 against 6.0e-7 there): an accumulator
-// is rounded 48 times a sub-tile instead of 64.
-namespace split {
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void parts(const float* x, bf16x8* p) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    f32x2 r = {x[e], x[e + 1]};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const bf16x2 b = __builtin_convertvector(r, bf16x2);
-      p[i][e] = b[0];
-      p[i][e + 1] = b[1];
-      r = r - __builtin_convertvector(b, f32x2);
-    }
-  }
-}
-__device__ __forceinline__ f32x16 mma(const bf16x8* a, const bf16x8* b, f32x16 c) {
-#pragma unroll
-  for (int o = 2; o >= 0; --o)
-#pragma unroll
-    for (int i = 0; i <= o; ++i) c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[o - i], c, 0, 0, 0);
-  return c;
-}
-}  // namespace split
-
-template <typename T, int D>
-constexpr int kFanMinWaves = sizeof(T) == 2 && D == 128 ? 2 : 1;
-template <typename T, int D>
-__global__ __launch_bounds__(kFanWaves * 64) __attribute__((amdgpu_waves_per_eu(kFanMinWaves<T, D>))) void attn_kernel_fan(AttnArgs a) {
-  constexpr int NW = kFanWaves;
-  using F = Frag<T, D>;
-  using P = typename F::P;
-  constexpr bool BF = sizeof(T) == 2;
-  constexpr int NDT = D / 32;
-  constexpr int kRB = D * (int)sizeof(T);          // bytes of one key row
-  constexpr int RS = D + 4;                        // row stride (floats) of a partial output in LDS
-  constexpr int kVBytes = BF ? NW * 2 * 32 * kRB : 0;  // two V sub-tiles per wave
-  constexpr int kOBytes = NW * 32 * RS * 4;        // one partial output per wave
-  __shared__ __align__(16) char lds[kVBytes > kOBytes ? kVBytes : kOBytes];
-  __shared__ float2 ml[NW * 32];
-
-  cev_plan_header ph;
-  if (!plan_ok(a, ph)) {
-    poison_output<T, D>(a);
-    return;
-  }
-  const int tid = threadIdx.x, lane = tid & 63, wave = uniform_i32(tid >> 6);
-  const int n = lane & 31, u = lane >> 5;
-  uint32_t item = blockIdx.x / (uint32_t)a.hkv;
-  const int kvh = (int)(blockIdx.x - item * (uint32_t)a.hkv);
-  int part = 0;
-  if (a.fan_parts > 1) {
-    part = (int)(item % (uint32_t)a.fan_parts);
-    item /= (uint32_t)a.fan_parts;
-  }
-  const int tile = (int)(item / (uint32_t)a.fan_subs), sub = (int)item - tile * a.fan_subs;
-  const int4 td = ((const int4*)(a.plan + ph.tiles_off))[2 * tile];
-  const int gs = __builtin_ctz(a.g);  // g is 1, 2, 4 or 8
-  const int sub_rows = 32 >> gs;
-  const int r0 = td.x + sub * sub_rows, nr = min(sub_rows, td.y - sub * sub_rows);
-  if (nr <= 0) return;
-  SlotRow sr;
-  sr.ok = (n >> gs) < nr && r0 + (n >> gs) < a.t;
-  sr.row = sr.ok ? r0 + (n >> gs) : 0;
-  sr.head = kvh * a.g + (n & (a.g - 1));
-
-  const T* const qrow = (const T*)a.q + (int64_t)sr.row * a.q_st + (int64_t)sr.head * a.q_sh;
-  F fr;                         // bf16
-  bf16x8 qp[BF ? 1 : D / 16][3];  // f32: the parts of q[16 st + 8 u ..]
-  auto load_q8 = [&](int st, float* x) {
-#pragma unroll
-    for (int e = 0; e < 8; e += 4) {
-      const f32x4 v = sr.ok ? *(const f32x4*)(qrow + 16 * st + 8 * u + e) : f32x4{};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[e + j] = v[j];
-    }
-  };
-  if constexpr (BF) {
-    fr.load_q(qrow, sr.ok, u);
-  } else {
-#pragma unroll
-    for (int st = 0; st < D / 16; ++st) {
-      float x[8];
-      load_q8(st, x);
-      split::parts(x, qp[st]);
-    }
-  }
-  int4 rv = ((const int4*)(a.plan + ph.rows_off))[sr.row];
-  if (!sr.ok) rv = make_int4(0, 0, -1, 0);
-  fan::Cursor cur;
-  cur.segs = (const int4*)(a.plan + ph.segs_off) + td.z;
-  cur.nseg = uniform_i32(td.w);
-  cur.s_cache = a.s_cache;
-  cur.t = a.t;
-  {
-    // the local keys that some row of these slots sees
-    int lo = rv.y > rv.x ? rv.x : INT32_MAX, hi = rv.y > rv.x ? rv.y : 0;
-    if (rv.z >= 0) {
-      lo = min(lo, rv.z);
-      hi = max(hi, rv.z + 1);
-    }
-    cur.lo = uniform_i32(fan::half_min(lo));
-    cur.hi = -uniform_i32(fan::half_min(-hi));
-  }
-  cur.start();
-  int c = wave, c_end = INT32_MAX;
-  if (a.fan_parts > 1) {
-    const int total = cur.total();
-    c = (int)((int64_t)part * total / a.fan_parts) + wave;
-    c_end = (int)((int64_t)(part + 1) * total / a.fan_parts);
-    cur.start();
-  }
-  KvSource<T> kvs;
-  kvs.init(a, kvh);
-
-  f32x16 o[NDT];
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
-  float m_run = -1e30f, l_run = 0.0f;
-  char* const vl = lds + wave * 2 * 32 * kRB;  // bf16: this wave's V sub-tiles
-  const int lds_v = (int)(size_t)(const __attribute__((address_space(3))) char*)vl;
-  int voff[NDT];
-  if constexpr (BF) {
-    const int i = lane & 15, rr = i >> 2, blk = 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) voff[dt] = (4 * u + rr) * kRB + (pipe::v_slot(4 * dt + blk, rr) << 4) + 8 * (i & 1);
-  }
-
-  // Loads of one sub-tile: K, 16 bytes of key row n per load, into kf; V into
-  // LDS buffer `buf` (bf16) or into vf (f32, issued on its own).  A sub-tile
-  // past the end has no valid key: its loads read no memory.
-  constexpr int kKLoads = kRB / 32, kVLoads = BF ? kRB / 32 : 0;
-  f32x4 kf[kKLoads];
-  float vf[BF ? 1 : 16][BF ? 1 : NDT];
-  __amdgpu_buffer_rsrc_t rk, rvs;
-  int kr, vr;
-  auto load_k = [&](const Chunk& x, int buf) {
-    kvs.rsrc(x, rk, rvs, kr, vr);
-#pragma unroll
-    for (int i = 0; i < kKLoads; ++i) {
-      // bf16: 8 values at 16 i + 8 u; f32: 4 values at 16 (i / 2) + 8 u + 4 (i % 2)
-      const int at = BF ? 32 * i + 16 * u : 64 * (i >> 1) + 32 * u + 16 * (i & 1);
-      kf[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, n * kr + at, 0, 0));
-    }
-    if constexpr (BF) {
-      constexpr int kRows = 1024 / kRB, kBlk = kRB / 16;  // rows of one 1 KB DMA, 16-byte blocks of a row
-#pragma unroll
-      for (int r = 0; r < kVLoads; ++r) {
-        const int vrow = kRows * r + lane / kBlk;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rvs, (__attribute__((address_space(3))) void*)(vl + buf * (32 * kRB) + 1024 * r), 16,
-                                                 vrow * vr + (pipe::v_slot(lane % kBlk, vrow) << 4), 0, 0, 0);
-      }
-    }
-  };
-  auto load_v = [&]() {
-    if constexpr (!BF) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-          vf[i][dt] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rvs, (8 * (i >> 2) + 4 * u + (i & 3)) * vr + (dt * 32 + n) * 4, 0, 0));
-    }
-  };
-  auto at = [&](int i, Chunk& x) {
-    x = Chunk{0, 0, 0};
-    return i < c_end && cur.seek(i, x);
-  };
-
-  // f32: an infinite value (or one above bf16's range) has no parts.  A wave
-  // that ends with anything non-finite walks its keys again on the f32 unit.
-  bool exact = false;
-  const int c_first = c;
-  Chunk ch, chn;
-  bool more;
-  int buf;
-  for (;;) {
-    more = at(c, ch);
-    buf = 0;
-    load_k(ch, 0);
-    load_v();
-    while (more) {
-      f32x16 s = f32x16{};
-#pragma unroll
-      for (int st = 0; st < D / 16; ++st) {
-        if constexpr (BF) {
-          fr.qk_mfma(__builtin_bit_cast(bf16x8, kf[st]), st, s);
-        } else {
-          float x[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] = kf[2 * st + (e >> 2)][e & 3];
-          if (!exact) {
-            bf16x8 kp[3];
-            split::parts(x, kp);
-            s = split::mma(kp, qp[st], s);
-          } else {
-            float q[8];
-            load_q8(st, q);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], q[e], s, 0, 0, 0);
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      c += NW;
-      more = at(c, chn);
-      load_k(chn, buf ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-      if (ch.local != 0 || ch.nvalid < 32) {
-        // Branch-free on purpose (see attn_kernel_seq).
-        const bool all_rows = ch.local == 0;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kk = 8 * (i >> 2) + 4 * u + (i & 3);
-          const int key = ch.key0 + kk;
-          const bool vis = (kk < ch.nvalid) & (all_rows | ((key >= rv.x) & (key < rv.y)) | (key == rv.z));
-          s[i] = vis ? s[i] : -INFINITY;
-        }
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
-      const float m_cand = pair_max(mx) * a.scale_log2;
-      const bool grow = m_cand > m_run + kRescale;
-      if (__ballot(grow)) {
-        const float m_new = grow ? m_cand : m_run;
-        const float alpha = fast_exp2(m_run - m_new);
-        m_run = m_new;
-        l_run *= alpha;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
-      }
-#pragma unroll
-      for (int i = 0; i < 16; ++i) s[i] = fast_exp2(__builtin_fmaf(s[i], a.scale_log2, -m_run));
-      P p;
-      F::make_p(s, p, l_run);
-      if constexpr (BF) {
-        // This sub-tile's V is in LDS once only the next one's loads are in
-        // flight.  The V^T reads go through asm (pipe::read_tr): the compiler
-        // would wait for the next sub-tile's DMA before each.
-        pipe::wait_vmcnt<kKLoads + kVLoads>();
-        asm volatile("" ::: "memory");
-        const int va = lds_v + buf * (32 * kRB);
-        constexpr int kGrp = 4;
-        pipe::i32x2 f[2][kGrp][2];
-        auto issue = [&](auto g_c) {
-          constexpr int G = decltype(g_c)::value;
-          static_for<kGrp>([&](auto e_c) {
-            constexpr int E = decltype(e_c)::value, J = G * kGrp + E;
-            constexpr int OFF = 16 * (J / NDT) * kRB;
-            f[G & 1][E][0] = pipe::read_tr<OFF>(va + voff[J % NDT]);
-            f[G & 1][E][1] = pipe::read_tr<OFF + 8 * kRB>(va + voff[J % NDT]);
-          });
-        };
-        issue(std::integral_constant<int, 0>{});
-        static_for<F::NPV / kGrp>([&](auto g_c) {
-          constexpr int G = decltype(g_c)::value;
-          static_for<kGrp>([&](auto e_c) {
-            constexpr int E = decltype(e_c)::value;
-            pipe::wait_tr<0>(f[G & 1][E][0], f[G & 1][E][1]);
-          });
-          if constexpr (G + 1 < F::NPV / kGrp) issue(std::integral_constant<int, G + 1>{});
-          static_for<kGrp>([&](auto e_c) {
-            constexpr int E = decltype(e_c)::value;
-            const bf16x4 lo = __builtin_bit_cast(bf16x4, f[G & 1][E][0]), hi = __builtin_bit_cast(bf16x4, f[G & 1][E][1]);
-            F::pv_mfma(bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}, G * kGrp + E, p, o);
-          });
-        });
-      } else {
-        if (!exact) {
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            float x[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = p.v[8 * h + e];
-            bf16x8 pp[3];
-            split::parts(x, pp);
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-#pragma unroll
-              for (int e = 0; e < 8; ++e) x[e] = vf[8 * h + e][dt];
-              bf16x8 vp[3];
-              split::parts(x, vp);
-              o[dt] = split::mma(vp, pp, o[dt]);
-            }
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[i][dt], p.v[i], o[dt], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        load_v();
-      }
-      ch = chn;
-      buf ^= 1;
-    }
-    if constexpr (BF) break;
-    float t = l_run * 0.0f + m_run * 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) t += o[dt][i] * 0.0f;
-    if (exact || !__any(!(t == 0.0f))) break;
-    exact = true;
-    c = c_first;
-    cur.start();
-    m_run = -1e30f;
-    l_run = 0.0f;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) o[dt] = f32x16{};
-  }
-  // loads past the end still write zeros into LDS: drain them
-  if (BF) pipe::wait_vmcnt<0>();
-
-  // ---- combine the waves' partials through LDS
-  const float l = pair_sum(l_run);
-  if (BF) __syncthreads();  // every wave is done with its V sub-tile
-  float* const ob = (float*)lds;
-#pragma unroll
-  for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4)
-      *(f32x4*)(ob + (wave * 32 + n) * RS + dt * 32 + 8 * q4 + 4 * u) = f32x4{o[dt][4 * q4], o[dt][4 * q4 + 1], o[dt][4 * q4 + 2], o[dt][4 * q4 + 3]};
-  if (u == 0) ml[wave * 32 + n] = make_float2(m_run, l);
-  // thread -> (slot, 8-column unit), the units of a slot side by side
-  constexpr int TPS = NW * 2, kUnits = D / 8 / TPS;
-  static_assert(D % (8 * TPS) == 0, "units split evenly");
-  const int slot = tid / TPS, tu = tid % TPS;
-  const int row = r0 + (slot >> gs), head = kvh * a.g + (slot & (a.g - 1));
-  const bool ok = (slot >> gs) < nr && row < a.t;
-  __syncthreads();
-  if (!ok) return;
-  float M = -INFINITY, L = 0.0f, w[NW];
-#pragma unroll
-  for (int i = 0; i < NW; ++i) M = fmaxf(M, ml[i * 32 + slot].x);
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const float2 v = ml[i * 32 + slot];
-    w[i] = fast_exp2(v.x - M);
-    L += w[i] * v.y;
-  }
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-#pragma unroll 1
-  for (int k = 0; k < kUnits; ++k) {
-    const int d = 8 * (tu + k * TPS);
-    float x[8] = {};
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      const float* pp = ob + (i * 32 + slot) * RS + d;
-      const f32x4 x0 = *(const f32x4*)pp, x1 = *(const f32x4*)(pp + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[e] += w[i] * x0[e];
-        x[4 + e] += w[i] * x1[e];
-      }
-    }
-    if (a.fan_parts > 1) {
-      const int64_t ri = record_index(a, row, head, part);  // fan_parts == n_splits here
-      T* rec = record_out<T, D>(a, ri) + d;
-      store_vec4<T>(rec, x);
-      store_vec4<T>(rec + 4, x + 4);
-      if (d == 0) record_ml<T, D>(a)[ri] = make_float2(M, L);
-      continue;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = BF ? x[e] * inv : (L > 0.0f ? x[e] / L : 0.0f);
-    if (a.has_gate) {
-      float gv[8];
-      const T* gp = (const T*)a.gate + (int64_t)row * a.g_st + (int64_t)head * a.g_sh + d;
-      load_vec4<T>(gp, gv);
-      load_vec4<T>(gp + 4, gv + 4);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = gate_value(x[e], gv[e], BF);
-    }
-    T* op = (T*)a.out + (int64_t)row * a.o_st + (int64_t)head * a.o_sh + d;
-    store_vec4<T>(op, x);
-    store_vec4<T>(op + 4, x + 4);
-  }
-}
-
 // Combines the parts of split tiles: for each (row, head),
 //   M = max_s m_s,  L = sum_s 2^(m_s - M) l_s,  O = sum_s 2^(m_s - M) O_s / L.
 // One wave per (row, head), kMergeWaves per workgroup.  Lane l reads the
@@ -2218,17 +1181,20 @@ __global__ __launch_bounds__(kMergeWaves * 64) void attn_merge_kernel(AttnArgs a
 // stagger: the bf16 d = 128 loop's form (attn_kernel_pipe's STAG).
 template <typename T, int D>
 int32_t launch(const AttnArgs& a, bool stagger, hipStream_t stream) {
-  const int64_t grid = (int64_t)a.n_tiles * (a.fan_parts > 0 ? (int64_t)a.fan_subs * a.fan_parts : a.n_splits) * a.hkv;
-  if (grid > INT32_MAX) return cev_fail(CEV_ERR_UNSUPPORTED, "grid of %lld workgroups is too large", (long long)grid);
-  if (a.fan_parts > 0)
-    hipLaunchKernelGGL((attn_kernel_fan<T, D>), dim3((unsigned)grid), dim3(kFanWaves * 64), 0, stream, a);
-  else if constexpr (sizeof(T) == 2 && D == 128)
-    hipLaunchKernelGGL((stagger ? attn_kernel_pipe<T, D, true> : attn_kernel_pipe<T, D, false>), dim3((unsigned)grid),
-                       dim3(kAttnWaves * 64), 0, stream, a);
-  else if constexpr (sizeof(T) == 2 && D == 256)
-    hipLaunchKernelGGL((attn_kernel_wide<T, D>), dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, stream, a);
-  else
-    hipLaunchKernelGGL((attn_kernel_seq<T, D>), dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, stream, a);
+  if (a.fan_parts > 0) {
+    int32_t rc = cev_attn_fan_launch(a, sizeof(T) == 2 ? CEV_BF16 : CEV_F32, D, stream);
+    if (rc) return rc;
+  } else {
+    const int64_t grid = (int64_t)a.n_tiles * a.n_splits * a.hkv;
+    if (grid > INT32_MAX) return cev_fail(CEV_ERR_UNSUPPORTED, "grid of %lld workgroups is too large", (long long)grid);
+    if constexpr (sizeof(T) == 2 && D == 128)
+      hipLaunchKernelGGL((stagger ? attn_kernel_pipe<T, D, true> : attn_kernel_pipe<T, D, false>), dim3((unsigned)grid),
+                         dim3(kAttnWaves * 64), 0, stream, a);
+    else if constexpr (sizeof(T) == 2 && D == 256)
+      hipLaunchKernelGGL((attn_kernel_wide<T, D>), dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_kernel_seq<T, D>), dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, stream, a);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return cev_fail(CEV_ERR_HIP, "packed attention launch: %s", hipGetErrorString(e));
   if ((a.fan_parts > 0 ? a.fan_parts : a.n_splits) > 1) {
