@@ -1320,6 +1320,37 @@ __device__ __forceinline__ bf16x4 read_tr(const __bf16* p) {
   return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4v*)p));
 }
 
+// Columns of x (the state or v_new, as a wave's lanes hold them) with a value
+// of kBig or more: scaled down with the same columns of S, out of reach of an
+// overflow before a row's factor divides by its norm (raw bf16 rows reach
+// 2^64, the factors 2^10) and of values that round to an infinite first part.
+// True if some column of the wave was; unscale() takes it back.
+constexpr float kBig = 0x1p50f;
+template <int N>
+__device__ __forceinline__ void multiply(f32x4v (&x)[N], float f) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = x[i] * f;
+}
+template <int N>
+__device__ __forceinline__ bool scale_columns(f32x4v (&x)[N], f32x4v (&S)[8], float& scale) {
+  float top = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) top = fmaxf(top, fabsf(x[i][e]));
+  if (__builtin_expect(__any(top >= kBig) == 0, 1)) return false;
+  top = fmaxf(top, __shfl_xor(top, 16, 64));
+  top = fmaxf(top, __shfl_xor(top, 32, 64));
+  scale = top >= kBig ? 0x1p-78f : 1.0f;
+  multiply(x, scale);
+  if ((void*)&x != (void*)&S) multiply(S, scale);
+  return true;
+}
+template <int N>
+__device__ __forceinline__ void unscale(f32x4v (&x)[N], float scale) {
+  multiply(x, 1.0f / scale);
+}
+
 template <typename T>
 __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2))) void gdn_fused_kernel(GdnArgs g) {
   constexpr bool BF = sizeof(T) == 2;
@@ -1429,13 +1460,22 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
       if constexpr (!BF) {
         // f32 models: the rows themselves are normalised (one rounding less
         // than a factor applied later); the factors are then 1.  x / n as
-        // x * (1/n) and one correction: rounded like the division.
+        // x * (1/n) and one correction: rounded like the division.  (A norm
+        // that overflowed divides to zero; the correction would be 0 * inf.)
         const float rq = 1.0f / nq, rk = 1.0f / nk;
+        const float cq = nq < INFINITY ? nq : 0.0f, ck = nk < INFINITY ? nk : 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float a = qv[e] * rq, b = kv[e] * rk;
-          qv[e] = __builtin_fmaf(__builtin_fmaf(-a, nq, qv[e]), rq, a) * 0.08838834764831845f;
-          kv[e] = __builtin_fmaf(__builtin_fmaf(-b, nk, kv[e]), rk, b);
+          qv[e] = __builtin_fmaf(__builtin_fmaf(-a, cq, qv[e]), rq, a) * 0.08838834764831845f;
+          kv[e] = __builtin_fmaf(__builtin_fmaf(-b, ck, kv[e]), rk, b);
+        }
+      } else if (__builtin_expect(__any(nq == INFINITY || nk == INFINITY) != 0, 0)) {
+        // a norm that overflowed divides to zero, before any product of the row does
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          qv[e] *= nq == INFINITY ? 0.0f : 1.0f;
+          kv[e] *= nk == INFINITY ? 0.0f : 1.0f;
         }
       }
       bf16x8 qp[3], kp[3];
@@ -1507,6 +1547,8 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
     f32x4v ks[4], qs[4];
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti) ks[ti] = qs[ti] = f32x4v{0, 0, 0, 0};
+    float s_scale = 1.0f;
+    bool s_big = false;
     auto state_step = [&](auto s_c) {
       constexpr int s = decltype(s_c)::value;
       if (!have_state) return;
@@ -1530,10 +1572,25 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
         qs[ti] = mma_parts<NA, 3>(a, sp, qs[ti]);
       }
     };
+    if (have_state) s_big = scale_columns(S, S, s_scale);
     state_step(std::integral_constant<int, 0>{});
     state_step(std::integral_constant<int, 1>{});
     state_step(std::integral_constant<int, 2>{});
     state_step(std::integral_constant<int, 3>{});
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) {
+      const f32x4 k4 = *(const f32x4*)(L.kf + 16 * ti + 4 * fq), q4 = *(const f32x4*)(L.qf + 16 * ti + 4 * fq);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ks[ti][e] *= k4[e];
+        qs[ti][e] *= q4[e];
+      }
+    }
+    if (__builtin_expect(s_big, 0)) {
+      unscale(S, s_scale);
+      unscale(ks, s_scale);
+      unscale(qs, s_scale);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's v is in LDS
     __syncthreads();  // ut, the diagonal inverses and intra are in LDS
 
@@ -1552,7 +1609,6 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
       vn[ti] = f32x4v{0, 0, 0, 0};
       if (ti >= nt) continue;
       const f32x4 b4 = *(const f32x4*)(L.betas + 16 * ti + 4 * fq), e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq);
-      const f32x4 k4 = *(const f32x4*)(L.kf + 16 * ti + 4 * fq);
       f32x4v lv = {0, 0, 0, 0};
 #pragma unroll
       for (int tj = 0; tj < ti; ++tj) {
@@ -1564,16 +1620,16 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const bool ok = t0 + 16 * ti + 4 * fq + e < g.t;
-        const float w = b4[e] * ((ok ? v_at(ti, e) : 0.0f) - e4[e] * (k4[e] * ks[ti][e])) - lv[e];
+        const float w = b4[e] * ((ok ? v_at(ti, e) : 0.0f) - e4[e] * ks[ti][e]) - lv[e];
         vn[ti] = mma16(a4[e], w, vn[ti]);
       }
     }
     if (c + 1 < g.n_chunks) load(t0 + kC);
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti) {
-      const f32x4 e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq), q4 = *(const f32x4*)(L.qf + 16 * ti + 4 * fq);
+      const f32x4 e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) out[ti][e] = e4[e] * (q4[e] * qs[ti][e]);
+      for (int e = 0; e < 4; ++e) out[ti][e] = e4[e] * qs[ti][e];
       if (ti >= nt) continue;
 #pragma unroll
       for (int tj = 0; tj <= ti; ++tj) {
@@ -1586,6 +1642,7 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
       const float decay = L.decay[0];
 #pragma unroll
       for (int ti = 0; ti < 8; ++ti) S[ti] = S[ti] * decay;
+      s_big = scale_columns(vn, S, s_scale);
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         if (2 * p >= nt) break;
@@ -1612,6 +1669,7 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
           S[ti] = mma_parts<NA, 3>(a, xp, S[ti]);
         }
       }
+      if (__builtin_expect(s_big, 0)) unscale(S, s_scale);
     }
 
     // ---- gated norm of the chunk's rows: 8 threads a row, 16 columns each

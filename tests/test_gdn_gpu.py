@@ -422,3 +422,36 @@ def test_fused_rows_vs_oracle(gpu, orc, bf16, batch, t, state):
     _say(f"fused {batch} x {t} bf16={bf16} state={state}: max|d| y {ey:.3g} state {es:.3g}")
     assert np.array_equal(to_np(co), rco)
     assert es <= F32_TOL and ey <= (BF16_TOL if bf16 else F32_TOL)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("batch,t", [(2, 40), (25, 65)])
+def test_large_finite_values_stay_finite(gpu, orc, bf16, batch, t):
+    """A state value above bf16's largest (its first bf16 part would round to
+    infinity), a value near it and, in f32, q and k rows whose squared norm
+    overflows (they divide to zero): finite results, as the oracle gives them.
+    The two large columns are compared relative to their largest value."""
+    w = configs.GdnWorkload("gdn-large", 31, bf16, batch, t, nk=2, nv=4)
+    inp = w.inputs()
+    s_in = 0.1 * np.random.default_rng(t).standard_normal((batch, 4, 128, 128)).astype(np.float32)
+    s_in[0, 0, 3, 7] = 3.4e38
+    inp["a"][0, :, 0] = inp["b"][0, :, 0] = -30.0  # that head keeps its state
+    inp["mixed"][1, t - 1, 4 * 128 + 9] = 3.38e38  # the last token's v, taken in whole by the state
+    inp["conv_w"][4 * 128 + 9] = [0, 0, 0, 1]
+    inp["a"][1, t - 1, 0], inp["b"][1, t - 1, 0] = -30.0, 30.0
+    if bf16:
+        inp["mixed"] = cev_hip.synth.round_bf16(inp["mixed"])
+    if not bf16:  # the last token of row 1 only, key head 1 (value heads 2 and 3)
+        inp["mixed"][1, t - 1, [128 + 5, 3 * 128 + 5]] = 3e19
+        inp["conv_w"][[128 + 5, 3 * 128 + 5], 3] = 1.0
+    y, _, so = _run_gpu(w, inp, gpu, s_in=to_dev(s_in, False, gpu))
+    with np.errstate(over="ignore"):
+        ry, _, rso = _run_oracle(orc, w, inp, s_in=s_in)
+    y, so = to_np(y), to_np(so)
+    assert np.isfinite(ry).all() and np.isfinite(rso).all()
+    assert np.isfinite(y).all() and np.isfinite(so).all()
+    for at in ((0, 0, slice(None), 7), (1, 0, slice(None), 9)):
+        assert np.abs(rso[at]).max() > 1e37
+        assert np.abs(so[at].astype(np.float64) - rso[at]).max() <= F32_TOL * np.abs(rso[at]).max()
+        so[at] = rso[at] = 0
+    assert np.abs(so - rso).max() <= F32_TOL and np.abs(y - ry).max() <= (BF16_TOL if bf16 else F32_TOL)
