@@ -112,13 +112,21 @@ void need_args(Py_ssize_t n, Py_ssize_t want) {
   if (n != want) raise_py(PyExc_TypeError, "expected " + std::to_string(want) + " arguments, got " + std::to_string(n));
 }
 
-// Runs an ABI call without the interpreter lock.
+// The interpreter lock let go of for its lifetime.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// Runs an ABI call without the interpreter lock.  The lock is held again
+// before an exception of fn's tensor accessors leaves.
 template <typename Fn>
 void call(Fn&& fn) {
   int32_t rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = fn();
-  Py_END_ALLOW_THREADS
+  {
+    Unlocked unlocked;
+    rc = fn();
+  }
   check(rc);
 }
 

@@ -33,6 +33,18 @@ def test_calls_check_tensors_before_any_launch(cev):
         cev_hip.gather_rows(z(4, 8), [0, 1], out=z(2, 8))
 
 
+def test_errors_inside_a_call_are_raised(cev):
+    """A tensor accessor that throws after the interpreter lock was let go
+    raises like any other (it used to end the process)."""
+    import torch
+    stream = type("Stream", (), {"cuda_stream": 0})()
+    x = torch.zeros(2, 64)
+    with pytest.raises(IndexError):
+        cev_hip.swiglu(x, x, out=torch.zeros(()), stream=stream)
+    with pytest.raises(IndexError):
+        cev_hip.gather_rows(x, out=torch.zeros(()), stream=stream)
+
+
 def test_tables_keep_their_blocks(cev):
     """A built table compiles from the builder's array; reading or replacing
     its block list makes the list the table."""
