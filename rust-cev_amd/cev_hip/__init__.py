@@ -400,7 +400,7 @@ def qknorm_rope_kv(q_in, k_in, v_in, w_q, w_k, pos, rot: Rotary, eps: float, q_o
     k_out / v_out (row i without slots), e.g. (t_or_capacity, hkv, d) views
     of head-major caches."""
     calls().qknorm_rope(q_in, k_in, w_q, w_k, pos, rot.cos, rot.sin, rot.rotary_dim, rot.n_pos, eps, plus_one, q_out, k_out, v_in, v_out,
-                        slots, n_slots, stream)
+                        slots, int(n_slots), stream)
     return q_out, k_out, v_out
 
 

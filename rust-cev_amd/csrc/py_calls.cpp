@@ -86,12 +86,12 @@ int dtype_code(const at::Tensor& t) {
   raise_cev(CEV_ERR_UNSUPPORTED, std::string("dtype torch.") + c10::toString(t.scalar_type()) + " not supported (float32, bfloat16)");
 }
 
-// The stream object's handle, or the current stream's.
+// The stream object's handle (None there is the default stream), or the current stream's.
 void* stream_of(PyObject* o) {
   if (o == Py_None) return (void*)c10::hip::getCurrentHIPStream().stream();
   PyObject* v = PyObject_GetAttrString(o, "cuda_stream");
   if (!v) throw Raised{};
-  const unsigned long long h = PyLong_AsUnsignedLongLong(v);
+  const unsigned long long h = v == Py_None ? 0 : PyLong_AsUnsignedLongLong(v);
   Py_DECREF(v);
   if (h == (unsigned long long)-1 && PyErr_Occurred()) throw Raised{};
   return (void*)(uintptr_t)h;
@@ -151,9 +151,11 @@ void rows_contiguous(const at::Tensor& t, const char* msg = "last dimension must
 PyObject* py_qknorm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&] {
     need_args(n, 18);
-    const at::Tensor &q_in = tensor(a[0], "q_in"), &k_in = tensor(a[1], "k_in"), &w_q = tensor(a[2], "w_q"), &w_k = tensor(a[3], "w_k"),
-                     &pos = tensor(a[4], "pos"), &cos = tensor(a[5], "cos"), &sin = tensor(a[6], "sin"), &q_out = tensor(a[11], "q_out"),
-                     &k_out = tensor(a[12], "k_out");
+    const at::Tensor &q_in = tensor(a[0], "q_in"), &k_in = tensor(a[1], "k_in"), &pos = tensor(a[4], "pos"),
+                     &q_out = tensor(a[11], "q_out"), &k_out = tensor(a[12], "k_out");
+    // (the ABI says which of these a call may go without)
+    const at::Tensor *w_q = tensor_or_none(a[2], "w_q"), *w_k = tensor_or_none(a[3], "w_k"), *cos = tensor_or_none(a[5], "cos"),
+                     *sin = tensor_or_none(a[6], "sin");
     const at::Tensor *v_in = tensor_or_none(a[13], "v_in"), *v_out = tensor_or_none(a[14], "v_out"), *slots = tensor_or_none(a[15], "slots");
     if (q_in.dim() != 3) raise_py(PyExc_ValueError, "q_in must be (t, heads, head_dim)");
     cev_qknorm_desc d;
@@ -302,10 +304,10 @@ PyObject* py_gdn(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (desc.b.len != (Py_ssize_t)sizeof(cev_gdn_desc)) raise_py(PyExc_TypeError, "desc must be a GdnDesc");
     cev_gdn_desc* d = (cev_gdn_desc*)desc.b.buf;
     const at::Tensor &mixed = tensor(a[1], "mixed"), &z = tensor(a[2], "z"), &b = tensor(a[3], "b"), &av = tensor(a[4], "a"),
-                     &conv_w = tensor(a[5], "conv_w"), &neg_a = tensor(a[6], "neg_a"), &dt_bias = tensor(a[7], "dt_bias"),
-                     &norm_w = tensor(a[8], "norm_w"), &y = tensor(a[11], "y"), &conv_out = tensor(a[12], "conv_out"),
-                     &s_out = tensor(a[13], "s_out"), &ws = tensor(a[14], "workspace");
-    const at::Tensor *conv_in = tensor_or_none(a[9], "conv_in"), *s_in = tensor_or_none(a[10], "s_in");
+                     &y = tensor(a[11], "y"), &conv_out = tensor(a[12], "conv_out"), &s_out = tensor(a[13], "s_out"),
+                     &ws = tensor(a[14], "workspace");
+    const at::Tensor *conv_w = tensor_or_none(a[5], "conv_w"), *neg_a = tensor_or_none(a[6], "neg_a"), *dt_bias = tensor_or_none(a[7], "dt_bias"),
+                     *norm_w = tensor_or_none(a[8], "norm_w"), *conv_in = tensor_or_none(a[9], "conv_in"), *s_in = tensor_or_none(a[10], "s_in");
     const auto want = d->dtype == CEV_BF16 ? at::kBFloat16 : at::kFloat;
     const char* const names[] = {"mixed", "z", "b", "a"};
     const at::Tensor* const in[] = {&mixed, &z, &b, &av};

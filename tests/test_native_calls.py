@@ -45,6 +45,22 @@ def test_errors_inside_a_call_are_raised(cev):
         cev_hip.gather_rows(x, out=torch.zeros(()), stream=stream)
 
 
+def test_missing_operands_are_the_abis_to_refuse(cev):
+    """None where only a pointer is passed on reaches the ABI's own check (a
+    call without q heads has no w_q)."""
+    import torch
+    z = lambda *s, dt=torch.float32: torch.zeros(*s, dtype=dt)  # noqa: E731
+    stream = type("Stream", (), {"cuda_stream": None})()
+    rot = type("R", (), dict(cos=z(4, 64), sin=z(4, 64), rotary_dim=128, n_pos=4))
+    with pytest.raises(CevError, match="null q") as e:
+        cev_hip.qknorm_rope(z(2, 2, 128), z(2, 1, 128), None, z(128), z(2, dt=torch.int32), rot, 1e-6, stream=stream)
+    assert e.value.code == -1
+    layer = cev_hip.GatedDeltaNet(1, 2, 2, 4, dtype=torch.float32, device="cpu")
+    with pytest.raises(CevError) as e:
+        layer(z(1, 2, 1024), z(1, 2, 512), z(1, 2, 4), z(1, 2, 4), None, z(4), z(4), z(128), stream=stream)
+    assert e.value.code == -1
+
+
 def test_tables_keep_their_blocks(cev):
     """A built table compiles from the builder's array; reading or replacing
     its block list makes the list the table."""
