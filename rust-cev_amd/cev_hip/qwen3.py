@@ -23,6 +23,11 @@ import numpy as np
 from . import (BlockTable, PackedAttention, Rotary, gather_rows, linear, qknorm_rope_kv, rms_norm, swiglu, upload_async)
 
 
+def _i32(a):
+    """a as int32, refusing Python integers that are out of its range."""
+    return np.ascontiguousarray(a, np.int32)
+
+
 class Qwen3Stack:
     def __init__(self, w, weights: dict, device, capacity: int, dtype=None, max_splits: int = 0):
         """w: a Qwen3StackWorkload (shapes); weights: {name: array} as made
@@ -84,8 +89,7 @@ class Qwen3Stack:
                                              L0["v"], self.max_splits)
         # the pass's tables and plan in one asynchronous copy (the host runs
         # ahead of the GPU; pageable copies made it wait for the last pass)
-        i32 = lambda a: np.asarray(a).astype(np.int32, copy=False)  # noqa: E731
-        ids, pos_d, slots_d, attn.plan.dev = upload_async([i32(tokens), i32(pos), i32(slots), attn.plan.host], self.device)
+        ids, pos_d, slots_d, attn.plan.dev = upload_async([_i32(tokens), _i32(pos), _i32(slots), attn.plan.host], self.device)
         if attn.plan.workspace_bytes:
             attn.plan.workspace = torch.empty(attn.plan.workspace_bytes, dtype=torch.uint8, device=self.device)
         gather_rows(self.embed, ids, out=x)
@@ -117,7 +121,7 @@ class Qwen3Stack:
         gathered rows only."""
         import torch
         x, h = xh
-        g, = upload_async([np.asarray(gather).astype(np.int32, copy=False)], self.device)
+        g, = upload_async([_i32(gather)], self.device)
         xg, hg = gather_rows(x, g), gather_rows(h, g)
         y = rms_norm(xg, self.norm, self.w.eps, h=hg, x_out=xg)
         return gather_rows(y, out_dtype=torch.float32)

@@ -61,6 +61,14 @@ def test_missing_operands_are_the_abis_to_refuse(cev):
     assert e.value.code == -1
 
 
+def test_token_ids_out_of_range_are_refused():
+    """A Python token id beyond int32 raises instead of wrapping around."""
+    from cev_hip.qwen3 import _i32
+    with pytest.raises(OverflowError):
+        _i32([1, 2**40])
+    assert _i32([1, 2]).dtype == np.int32 and _i32(np.array([3, 4], np.int64)).tolist() == [3, 4]
+
+
 def test_tables_keep_their_blocks(cev):
     """A built table compiles from the builder's array; reading or replacing
     its block list makes the list the table."""
