@@ -308,9 +308,9 @@ int32_t cev_debias_scores(int32_t n_questions, int32_t n_variants, const int32_t
 /* Linear layers and row gathers (the candle ops around the attention call
  * in the device-resident stack and the readouts).
  *
- * cev_blas is a hipBLASLt context for products of more than 8 rows; it
- * caches one algorithm per problem shape.  Use a handle from one thread at a
- * time. */
+ * cev_blas is a hipBLASLt context for the library's part of the products of
+ * more than 8 rows; it caches one algorithm per problem shape.  Use a handle
+ * from one thread at a time. */
 typedef void* cev_blas;
 int32_t cev_blas_create(cev_blas* handle);
 int32_t cev_blas_destroy(cev_blas handle);
@@ -323,10 +323,12 @@ int32_t cev_blas_destroy(cev_blas handle);
  * row stride ldy, all row-major; x and w in `dtype`, y in out_dtype (CEV_F32
  * or dtype); f32 accumulation, one rounding to the output dtype.  m <= 8
  * runs this library's own kernel (handle may be NULL, no workspace); larger
- * m a hipBLASLt GEMM on `handle` with the caller's workspace
- * (CEV_LINEAR_WORKSPACE_BYTES recommended; 0 allowed).  x and w must be
- * 16-byte aligned with ldx, ldw multiples of 8 (bf16) or 4 (f32) elements;
- * for m > 8 the same holds for y and ldy in the output dtype. */
+ * m need a handle and use the caller's workspace (CEV_LINEAR_WORKSPACE_BYTES
+ * recommended; 0 allowed): f32 products large enough to fill the GPU run this
+ * library's own kernel too (sums of parts of k in the workspace), all others
+ * are a hipBLASLt GEMM.  Calls sharing one workspace must not overlap.  x and
+ * w must be 16-byte aligned with ldx, ldw multiples of 8 (bf16) or 4 (f32)
+ * elements; for m > 8 the same holds for y and ldy in the output dtype. */
 #define CEV_LINEAR_WORKSPACE_BYTES ((size_t)32 << 20)
 int32_t cev_linear(cev_blas handle, int32_t dtype, int32_t out_dtype, int64_t m, int64_t n, int64_t k, const void* x, int64_t ldx,
                    const void* w, int64_t ldw, float alpha, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,

@@ -458,16 +458,24 @@ def debias_scores(logits, order, span_begin, span_len, n_options, calib=None, st
 
 
 class Blas:
-    """A cev_blas context (hipBLASLt, cached algorithms) and its workspace on
-    one device; Blas.on(device) keeps one per device."""
+    """A cev_blas context (hipBLASLt, cached algorithms) and a workspace on
+    one device; Blas.on(device) keeps one per device.  The workspace belongs
+    to the calls that pass this object to linear(): those of one stream at a
+    time."""
     _per_device: dict = {}
 
     def __init__(self, device):
-        torch = _torch()
         h = C.c_void_p()
         check(lib().cev_blas_create(C.byref(h)))
         self.handle = h
-        self.workspace = torch.empty(CEV_LINEAR_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
+        self._device, self._workspace = device, None
+
+    @property
+    def workspace(self):
+        if self._workspace is None:
+            torch = _torch()
+            self._workspace = torch.empty(CEV_LINEAR_WORKSPACE_BYTES, dtype=torch.uint8, device=self._device)
+        return self._workspace
 
     @classmethod
     def on(cls, device) -> "Blas":
@@ -488,13 +496,18 @@ class Blas:
 def linear(x, w, out=None, alpha: float = 1.0, out_dtype=None, blas: Optional[Blas] = None, stream=None):
     """out = out_dtype(alpha * x @ w.T) for x (m, k), w (n, k): candle's bias-free
     Linear::forward (qwen3.rs:175-178, :229-233), the code head (engine.rs:463)
-    and the d3 readout (hybrid.rs:657, alpha = 1 / temperature)."""
+    and the d3 readout (hybrid.rs:657, alpha = 1 / temperature).  Without blas
+    a call of more than 8 rows takes its workspace from torch's allocator for
+    its stream, so calls on several streams may overlap."""
     m = x.shape[0]
     if out is None:
         out = _torch().empty((m, w.shape[0]), dtype=x.dtype if out_dtype is None else out_dtype, device=x.device)
-    if blas is None and m > 8:
-        blas = Blas.on(x.device)
-    calls().linear(x, w, out, alpha, None if blas is None else blas.handle.value, None if blas is None else blas.workspace, stream)
+    if blas is not None:
+        calls().linear(x, w, out, alpha, blas.handle.value, blas.workspace, 0, stream)
+    elif m > 8:
+        calls().linear(x, w, out, alpha, Blas.on(x.device).handle.value, None, CEV_LINEAR_WORKSPACE_BYTES, stream)
+    else:
+        calls().linear(x, w, out, alpha, None, None, 0, stream)
     return out
 
 

@@ -13,7 +13,8 @@
 //
 // Row counts of up to kRowsSmall (decode-like readouts, the code head of a
 // few questions) run on this file's own kernel, which streams every weight
-// row once; larger products are plain library GEMMs (hipBLASLt), f32
+// row once, and f32 products that fill the chip on its split kernel (bf16
+// matrix cores); all others are plain library GEMMs (hipBLASLt).  f32
 // accumulation, the result rounded once to the output dtype as candle's
 // matmul does.
 #include <hipblaslt/hipblaslt-ext.hpp>

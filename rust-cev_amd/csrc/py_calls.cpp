@@ -14,6 +14,8 @@
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 
 #include <string>
@@ -257,10 +259,27 @@ PyObject* py_swiglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
-// linear(x, w, out, alpha, handle, workspace, stream)
+// A device buffer of one call, from torch's allocator for the call's stream:
+// given back once the call is queued, so only later work of that stream gets
+// the memory, and a captured call's belongs to its graph.
+struct CallBuffer {
+  void* p = nullptr;
+  CallBuffer(const at::Tensor& on, size_t bytes, void* stream) {
+    if (bytes == 0 || !on.is_cuda()) return;
+    const c10::DeviceGuard guard(on.device());
+    p = c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, (hipStream_t)stream);
+  }
+  ~CallBuffer() {
+    if (p) c10::hip::HIPCachingAllocator::raw_delete(p);
+  }
+  CallBuffer(const CallBuffer&) = delete;
+  CallBuffer& operator=(const CallBuffer&) = delete;
+};
+
+// linear(x, w, out, alpha, handle, workspace, workspace_bytes, stream): without a workspace one of workspace_bytes is taken for the call
 PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return guarded([&] {
-    need_args(n, 7);
+    need_args(n, 8);
     const at::Tensor &x = tensor(a[0], "x"), &w = tensor(a[1], "w"), &out = tensor(a[2], "out");
     const at::Tensor* ws = tensor_or_none(a[5], "workspace");
     if (x.dim() != 2) raise_py(PyExc_ValueError, "x must be (m, k)");
@@ -270,10 +289,14 @@ PyObject* py_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int odt = dtype_code(out);
     const float alpha = (float)as_double(a[3]);
     const cev_blas handle = a[4] == Py_None ? nullptr : (cev_blas)(uintptr_t)as_int(a[4]);
-    void* const s = stream_of(a[6]);
+    void* const s = stream_of(a[7]);
+    size_t bytes = ws ? (size_t)ws->numel() : (size_t)as_int(a[6]);
+    const CallBuffer own(x, ws ? 0 : bytes, s);
+    void* const buffer = ws ? ptr(ws) : own.p;
+    if (!buffer) bytes = 0;
     call([&] {
       return api.linear(handle, dt, odt, x.size(0), w.size(0), x.size(1), ptr(x), x.stride(0), ptr(w), w.stride(0), alpha, ptr(out),
-                        out.stride(0), ptr(ws), ws ? (size_t)ws->numel() : 0, s);
+                        out.stride(0), buffer, bytes, s);
     });
   });
 }

@@ -362,6 +362,33 @@ def test_split_f32_product(gpu, m, n, k):
     assert (got - want).norm() / want.norm() < 3e-6
 
 
+def test_products_on_two_streams_do_not_share_sums(gpu):
+    """f32 products whose parts of k are summed through a workspace, queued on
+    two streams at once, with and without a current stream: each call has a
+    workspace of its own stream's."""
+    import torch
+
+    import cev_hip
+    m, n, k = 912, 2048, 6144
+    g = torch.Generator().manual_seed(12)
+    x = [torch.randn(m, k, generator=g).to(gpu) for _ in range(2)]
+    w = torch.randn(n, k, generator=g).to(gpu)
+    want = [cev_hip.linear(v, w) for v in x]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    out = [[torch.empty_like(want[0]) for _ in range(8)] for _ in range(2)]
+    torch.cuda.synchronize()
+    for i in range(8):
+        for j in range(2):
+            if i % 2:
+                cev_hip.linear(x[j], w, out=out[j][i], stream=streams[j])
+            else:
+                with torch.cuda.stream(streams[j]):
+                    cev_hip.linear(x[j], w, out=out[j][i])
+    torch.cuda.synchronize()
+    for j in range(2):
+        assert all(torch.equal(o, want[j]) for o in out[j])
+
+
 def test_split_f32_product_keeps_infinities(gpu):
     """Values without bf16 parts (infinite, or above bf16's range) give what
     plain f32 products give: their tile is computed again one by one."""
