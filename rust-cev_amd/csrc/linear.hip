@@ -122,10 +122,13 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_rows_kernel(LinArgs a) 
 // ---------------------------------------------------------------------------
 // f32 products of more than kRowsSmall rows on the bf16 matrix cores.
 // Every f32 value is split into three bf16 parts (round to nearest each; the
-// parts' sum is the value) and six of the nine part products are summed in
-// f32: the three dropped ones are below 2^-26 of the product each.  Six bf16
-// products cost 6/16 of the f32 unit's time, and the accumulator is rounded
-// once per 16 products of a part pair instead of once per 2.
+// parts' sum is the value, the second at most 2^-8 and the third 2^-17 of it)
+// and six of the nine part products are summed in f32.  Of the three dropped
+// ones the two larger are at most 2^-25 of the product each, all three 2^-24.
+// Six bf16 products cost 6/16 of the f32 unit's time.  The products of the
+// first parts have an accumulator of their own, rounded once per 16 products
+// (the f32 unit's once per 2), and the five small ones, whose roundings weigh
+// 2^-8 as much, another; they meet at the end.
 //
 // A workgroup of eight waves computes a 128 x 128 tile of y, each wave 64 x 32
 // of it on 32x32x16 MFMAs.  A 32-deep slice of x and w goes through registers
@@ -134,13 +137,14 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_rows_kernel(LinArgs a) 
 // three planes of 64-byte rows, 16-byte piece c of row r at c ^ (r / 4 % 4) so
 // that a fragment read touches every bank.
 // What bounds it: a slice takes 3000 clocks a CU where its MFMAs need 1536 and
-// its LDS traffic (195 KB) 1500; 185-193 TFLOP/s of f32 products at 2048 rows
-// (library 131-149).  Tried: one buffer and one slice ahead 134 us at
+// its LDS traffic (195 KB) 1500; 195-202 TFLOP/s of f32 products at 2048 rows
+// (library 146-150).  Tried: one buffer and one slice ahead 134 us at
 // 200 x 4096 x 2048 (72 now); four waves a tile 89; 64-wide tiles 113 against
 // 95 at 912 x 4096 x 2048; 256 x 128 tiles 4-6 % faster at 2048 rows and half
 // a round short at 912.
-// Error against f64, N(0,1) x 0.02 N(0,1): 7.0e-7 at k = 2048 (library
-// 8.1e-7), 1.24e-6 at 6144 (1.40e-6).
+// Error against f64, N(0,1) x 0.02 N(0,1): 2.7e-7 at k = 2048 (library
+// 8.1e-7), 4.9e-7 at 6144 (1.40e-6); with one accumulator for all six 7.0e-7
+// and 1.24e-6 at the same times.
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
@@ -206,11 +210,11 @@ __global__ __launch_bounds__(kSplitWaves * 64) __attribute__((amdgpu_waves_per_e
     return *(const bf16x8*)(lds + buf * kBuf + plane * kPlane + r * kSliceK + ((((2 * ks + u) ^ (r >> 2)) & 3) << 3));
   };
 
-  f32x16 acc[TM][TN];
+  f32x16 acc[TM][TN], low[TM][TN];  // products of the first parts, and of the others
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+    for (int j = 0; j < TN; ++j) acc[i][j] = low[i][j] = f32x16{};
   // this part's slices of k
   const int all = (int)((a.k + kSliceK - 1) / kSliceK);
   const int s0 = (int)((int64_t)part * all / parts), s1 = (int)((int64_t)(part + 1) * all / parts);
@@ -231,7 +235,6 @@ __global__ __launch_bounds__(kSplitWaves * 64) __attribute__((amdgpu_waves_per_e
 #pragma unroll
       for (int j = 0; j < TN; ++j) fw[j][p] = frag(buf, p, BM + wn * WN + 32 * j + n32, ks);
     }
-    // small products first
 #pragma unroll
     for (int o = 2; o >= 0; --o)
 #pragma unroll
@@ -239,7 +242,10 @@ __global__ __launch_bounds__(kSplitWaves * 64) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i][p], fw[j][o - p], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < TN; ++j) {
+            f32x16& sum = o > 0 ? low[i][j] : acc[i][j];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i][p], fw[j][o - p], sum, 0, 0, 0);
+          }
   };
   // Slice sl is multiplied while slice sl + 1 is split into the other buffer
   // (past the end: a repeat of the last columns, counted as zero) and slices
@@ -263,6 +269,11 @@ __global__ __launch_bounds__(kSplitWaves * 64) __attribute__((amdgpu_waves_per_e
     step(sl, std::integral_constant<int, 0>{});
     if (sl + 1 < s1) step(sl + 1, std::integral_constant<int, 1>{});
   }
+
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
 
   // An infinite value (or one above bf16's range) has no parts: x - bf16(x) is
   // not a number.  A wave whose quarter came out non-finite anywhere computes
