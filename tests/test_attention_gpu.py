@@ -59,10 +59,18 @@ def _check_blocks(gl, ol, blocks, tol, rows=None):
     return worst
 
 
-def test_c1_f32_end_to_end(gpu, orc):
+def _replan(gl, max_splits):
+    """The layer's attention planned with max_splits (1: the 256-slot kernels)."""
+    gl.attn = cev_hip.PackedAttention(gl.q, gl.k, gl.table, k_cache=gl.pk, s_cache=gl.w.prefix, has_gate=gl.w.gated, out=gl.out,
+                                      gate=gl.gate, v_new=gl.v, v_cache=gl.pv, max_splits=max_splits)
+
+
+@pytest.mark.parametrize("max_splits", [0, 1])
+def test_c1_f32_end_to_end(gpu, orc, max_splits):
     w = configs.c1()
-    _say(f"test c1: t={w.t} P={w.prefix} hq={w.hq} hkv={w.hkv}")
+    _say(f"test c1: t={w.t} P={w.prefix} hq={w.hq} hkv={w.hkv} max_splits={max_splits}")
     gl = GpuLayer(w, gpu)
+    _replan(gl, max_splits)
     ol = OracleLayer(orc, w, gl.np_inputs)
     gl.forward()
     # K1 reproduces the reference op order exactly
@@ -127,7 +135,7 @@ def test_c4_bidirectional_gated_full_row(gpu, orc):
         _check_blocks(gl, ol, [0], BF16_TOL, rows=(r0, 64))
 
 
-def _d3_check(gpu, orc, w, tol):
+def _d3_check(gpu, orc, w, tol, max_splits=0):
     """GPU: K1 + K2 over the whole row, then o_proj of the last position and
     the readout (D3Readout through cev_linear / cev_gather_rows).  Oracle:
     the same chain from the same inputs (attention of the last row by the
@@ -135,6 +143,7 @@ def _d3_check(gpu, orc, w, tol):
     import torch
     from oracle.readout import d3_readout
     gl = GpuLayer(w, gpu)
+    _replan(gl, max_splits)
     ol = OracleLayer(orc, w, gl.np_inputs)
     gl.forward()
     torch.cuda.synchronize()
@@ -164,8 +173,9 @@ def test_c4_d3_readout_full_row(gpu, orc):
     _d3_check(gpu, orc, configs.c4(), BF16_TOL)
 
 
-def test_d3_readout_f32_small(gpu, orc):
-    _d3_check(gpu, orc, configs.d3_f32(), F32_TOL)
+@pytest.mark.parametrize("max_splits", [0, 1])
+def test_d3_readout_f32_small(gpu, orc, max_splits):
+    _d3_check(gpu, orc, configs.d3_f32(), F32_TOL, max_splits)
 
 
 def test_linear_shapes_against_numpy(gpu, orc):
@@ -238,8 +248,14 @@ SMALL = [
 ]
 
 
+# max_splits = 1 keeps a call on the 256-slot kernels; with 0 the planner
+# takes these small ones to the small-launch kernel
+BOTH_FORMS = pytest.mark.parametrize("max_splits", [0, 1])
+
+
+@BOTH_FORMS
 @pytest.mark.parametrize("case", range(len(SMALL)))
-def test_small_packed_passes(gpu, orc, case):
+def test_small_packed_passes(gpu, orc, case, max_splits):
     """Multi-plan passes with tails, ragged blocks, every GQA group size and
     both head dims, against the oracle over the reference's dense mask."""
     bf, hq, hkv, d, plans, items = SMALL[case]
@@ -255,7 +271,8 @@ def test_small_packed_passes(gpu, orc, case):
     kc = rnd(rng.standard_normal((hkv, max(s_cache, 1), d)).astype(np.float32))[:, :s_cache]
     vc = rnd(rng.standard_normal((hkv, max(s_cache, 1), d)).astype(np.float32))[:, :s_cache]
     out = cev_hip.packed_attention(to_dev(q, bf, gpu), to_dev(kn, bf, gpu), to_dev(vn, bf, gpu), tab,
-                                   k_cache=to_dev(kc, bf, gpu) if s_cache else None, v_cache=to_dev(vc, bf, gpu) if s_cache else None)
+                                   k_cache=to_dev(kc, bf, gpu) if s_cache else None, v_cache=to_dev(vc, bf, gpu) if s_cache else None,
+                                   max_splits=max_splits)
     got = to_np(out)
     kall = np.concatenate([kc, kn.transpose(1, 0, 2)], axis=1)
     vall = np.concatenate([vc, vn.transpose(1, 0, 2)], axis=1)
@@ -325,20 +342,23 @@ def test_softmax_max_moves(gpu, orc, shape, max_splits):
                                                   ("bf16", 16, 4, 256, True), ("f32", 16, 8, 128, False), ("f32", 8, 2, 128, True)])
 @pytest.mark.parametrize("case", ["one_key", "ragged", "tail", "split", "bidir", "scattered"])
 def test_small_launches_vs_oracle(gpu, orc, dtype, hq, hkv, d, gated, case):
-    """The small-launch kernel at its edges: one token without a prefix (one
-    key, three idle waves), groups cut inside blocks, a tail span, several
+    """The small-launch kernel at its edges: one token of as few keys as the
+    planner takes there (one in bf16, d = 128, for three idle waves; two and
+    34 in f32 and at d = 256), groups cut inside blocks, a tail span, several
     parts of the key stream with remainders, bidirectional rows with padded
     ones, and more segments per tile than a wave has lanes."""
     bf = dtype == "bf16"
     cap = 0
     if case == "one_key":
-        tab = cev_hip.BlockTable.from_rows(1, 1, 0, causal=True)
+        past = 0 if bf and d == 128 else 33 if bf else 1
+        tab, _, _ = cev_hip.BlockTable.from_plans([(past, past, past)], [(0, 1)])
     elif case == "ragged":
         tab, _, _ = cev_hip.BlockTable.from_plans([(33, 33, 33)], [(0, n) for n in (1, 31, 32, 33, 7, 65)])
     elif case == "tail":
         tab, _, _ = cev_hip.BlockTable.from_plans([(129, 226, 129)], [(0, 5), (0, 40)])
     elif case == "split":
-        tab, _, _ = cev_hip.BlockTable.from_plans([(1427, 1427, 1427)], [(0, 19), (0, 22)])
+        past = 300 if not bf else 1427 if d == 128 else 500
+        tab, _, _ = cev_hip.BlockTable.from_plans([(past, past, past)], [(0, 19), (0, 22)])
     elif case == "bidir":
         tab = cev_hip.BlockTable.from_rows(4, 43, 0, causal=False, lengths=[43, 17, 1, 0])
     else:  # one-token questions in every other slot: one segment each
@@ -356,7 +376,7 @@ def test_small_launches_vs_oracle(gpu, orc, dtype, hq, hkv, d, gated, case):
     op = cev_hip.PackedAttention(qd, knd, tab, s_cache=s, has_gate=gated, gate=gd if gated else None, v_new=vnd, **args)
     parts = int(op.plan.header()[18])
     _say(f"small launch {case} {dtype} hq {hq} hkv {hkv} d {d}: tiles {op.plan.n_tiles}, parts {parts} of {op.plan.n_splits}")
-    assert parts >= 1 or case in ("one_key", "split"), "the planner should run this table on the small-launch kernel"
+    assert parts > (1 if case == "split" else 0), "the planner should run this table on the small-launch kernel"
     got = to_np(op(qd, knd, vnd, gate=gd if gated else None, **args))
     mask = tab.to_dense_mask()
     K, V = np.concatenate([kc, kn.transpose(1, 0, 2)], 1), np.concatenate([vc, vn.transpose(1, 0, 2)], 1)
@@ -439,8 +459,9 @@ def test_packed_rows_equal_each_row_alone_d256(gpu):
         assert np.array_equal(to_np(alone), packed[r0:r0 + L])
 
 
+@BOTH_FORMS
 @pytest.mark.parametrize("d", [128, 256])
-def test_poisoned_invisible_keys_are_never_read(gpu, orc, d):
+def test_poisoned_invisible_keys_are_never_read(gpu, orc, d, max_splits):
     """A row never reads another plan's K/V.  Per plan p: NaN in every other
     plan's past (cache keys), in the K/V of every new token another plan
     owns, and in keys past the end of the cache must leave plan p's rows
@@ -467,7 +488,8 @@ def test_poisoned_invisible_keys_are_never_read(gpu, orc, d):
     vc = orc.round_bf16(rng.standard_normal((hkv, s + pad, d)).astype(np.float32))
     qd = to_dev(q, bf, gpu)
     clean = to_np(cev_hip.packed_attention(qd, to_dev(kn, bf, gpu), to_dev(vn, bf, gpu), tab,
-                                           k_cache=to_dev(kc, bf, gpu)[:, :s], v_cache=to_dev(vc, bf, gpu)[:, :s]))
+                                           k_cache=to_dev(kc, bf, gpu)[:, :s], v_cache=to_dev(vc, bf, gpu)[:, :s],
+                                           max_splits=max_splits))
     assert np.isfinite(clean).all()
     for p in range(len(plans)):
         kcp, vcp, knp, vnp = kc.copy(), vc.copy(), kn.copy(), vn.copy()
@@ -481,7 +503,8 @@ def test_poisoned_invisible_keys_are_never_read(gpu, orc, d):
         kcp[:, s:] = np.nan
         vcp[:, s:] = np.nan
         got = to_np(cev_hip.packed_attention(qd, to_dev(knp, bf, gpu), to_dev(vnp, bf, gpu), tab,
-                                             k_cache=to_dev(kcp, bf, gpu)[:, :s], v_cache=to_dev(vcp, bf, gpu)[:, :s]))
+                                             k_cache=to_dev(kcp, bf, gpu)[:, :s], v_cache=to_dev(vcp, bf, gpu)[:, :s],
+                                             max_splits=max_splits))
         torch.cuda.synchronize()
         mine = owner == p
         _say(f"poisoned run for plan {p}, d={d}: {int(mine.sum())} rows checked")
@@ -512,7 +535,8 @@ def test_stale_device_plan_gives_nan_not_stale_rows(gpu):
     assert torch.isnan(out.float()).all()
 
 
-def test_rows_outside_every_block_are_untouched(gpu):
+@BOTH_FORMS
+def test_rows_outside_every_block_are_untouched(gpu, max_splits):
     import torch
     t, hq, hkv, d, s = 100, 8, 2, 128, 30
     B = cev_hip.BlockTable.block
@@ -521,7 +545,7 @@ def test_rows_outside_every_block_are_untouched(gpu):
     k = torch.randn(t, hkv, d, device=gpu).to(torch.bfloat16)
     kc = torch.randn(hkv, s, d, device=gpu).to(torch.bfloat16)
     out = torch.full((t, hq, d), 7.0, device=gpu, dtype=torch.bfloat16)
-    cev_hip.packed_attention(q, k, k, tab, k_cache=kc, v_cache=kc, out=out)
+    cev_hip.packed_attention(q, k, k, tab, k_cache=kc, v_cache=kc, out=out, max_splits=max_splits)
     o = to_np(out)
     assert (o[:10] == 7).all() and (o[30:60] == 7).all() and (o[65:] == 7).all()
     assert not (o[10:30] == 7).all()
@@ -575,7 +599,8 @@ def test_stale_device_plan_split_gives_nan(gpu):
     assert torch.isnan(out.float()).all()
 
 
-def test_bidirectional_padded_rows(gpu, orc):
+@BOTH_FORMS
+def test_bidirectional_padded_rows(gpu, orc, max_splits):
     bf, t, hq, hkv, d = True, 40, 8, 2, 256
     lengths = [40, 17, 1, 0]
     tab = cev_hip.BlockTable.from_rows(len(lengths), t, 0, causal=False, lengths=lengths)
@@ -584,7 +609,7 @@ def test_bidirectional_padded_rows(gpu, orc):
     q = orc.round_bf16(rng.standard_normal((n, hq, d)).astype(np.float32))
     k = orc.round_bf16(rng.standard_normal((n, hkv, d)).astype(np.float32))
     v = orc.round_bf16(rng.standard_normal((n, hkv, d)).astype(np.float32))
-    got = to_np(cev_hip.packed_attention(to_dev(q, bf, gpu), to_dev(k, bf, gpu), to_dev(v, bf, gpu), tab))
+    got = to_np(cev_hip.packed_attention(to_dev(q, bf, gpu), to_dev(k, bf, gpu), to_dev(v, bf, gpu), tab, max_splits=max_splits))
     mask = orc.bidirectional_mask(t, lengths)
     for r in range(len(lengths)):
         sl = slice(r * t, (r + 1) * t)
