@@ -116,7 +116,11 @@ typedef struct {
    * over several workgroups when there are too few tiles to fill the GPU),
    * 1 disables it, n > 1 caps the parts per tile at n.  Split parts write
    * partial results to the workspace and a merge pass combines them, so
-   * results can differ from an unsplit run in the last bits. */
+   * results can differ from an unsplit run in the last bits.  Unless it is
+   * 1 the planner also chooses, by modelled times, between the kernels of
+   * 256 query slots a workgroup and one of 32 for launches with few rows,
+   * whose sums are in another order; 1 keeps every call of any row count on
+   * the former, one walk over a row's keys in stream order. */
   int32_t max_splits;
   int32_t reserved;
 } cev_attn_desc;
@@ -248,6 +252,10 @@ typedef struct cev_gdn_desc {
 int32_t cev_gdn_desc_init(cev_gdn_desc* d, int32_t dtype, int32_t batch, int32_t t, int32_t n_k_heads, int32_t n_v_heads,
                           int32_t head_k_dim, int32_t head_v_dim, int32_t conv_kernel, float eps);
 int32_t cev_gdn_workspace_size(const cev_gdn_desc* d, size_t* bytes);
+/* Which kernels a call runs after the conv: *fused = 1 one kernel for each
+ * (row, value head), 0 prep, scan and norm (host only; the two forms' results
+ * differ in the last bits). */
+int32_t cev_gdn_form(const cev_gdn_desc* d, int32_t* fused);
 
 /* One layer for B rows of T tokens.  mixed, z, b, a, conv_w (conv_dim, K),
  * conv_in and y are in the model dtype; neg_a = -exp(A_log), dt_bias and
@@ -333,6 +341,10 @@ int32_t cev_blas_destroy(cev_blas handle);
 int32_t cev_linear(cev_blas handle, int32_t dtype, int32_t out_dtype, int64_t m, int64_t n, int64_t k, const void* x, int64_t ldx,
                    const void* w, int64_t ldw, float alpha, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,
                    cev_stream stream);
+
+/* Which kernel a product of the sizes runs: *form = 0 the small-row kernel, p >= 1
+ * the f32 split kernel over p parts of k, -1 hipBLASLt (host only). */
+int32_t cev_linear_form(int32_t dtype, int64_t m, int64_t n, int64_t k, size_t workspace_bytes, int32_t* form);
 
 /* out[i] = out_dtype(table[ids[i]]) for i < n, rows of `width` elements:
  * Embedding::forward's rows (qwen3.rs:288-293), index_select of the answer

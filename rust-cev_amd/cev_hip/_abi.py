@@ -104,6 +104,7 @@ SIGNATURES = {
     "cev_rope_table": (i32, [C.c_double, i32, i32, i32, P, P]),
     "cev_gdn_desc_init": (i32, [C.POINTER(GdnDesc), i32, i32, i32, i32, i32, i32, i32, i32, C.c_float]),
     "cev_gdn_workspace_size": (i32, [C.POINTER(GdnDesc), C.POINTER(C.c_size_t)]),
+    "cev_gdn_form": (i32, [C.POINTER(GdnDesc), Pi32]),
     "cev_gdn_forward": (i32, [C.POINTER(GdnDesc), P, P, P, P, P, P, P, P, P, P, P, P, P, P, C.c_size_t, P]),
     "cev_rms_norm": (i32, [i32, i64, i32, P, i64, P, i64, P, i64, P, C.c_float, i32, P, i64, P]),
     "cev_rms_norm_seq": (i32, [i32, i64, i32, P, i64, P, i64, P, i64, P, C.c_float, i32, P, i64, P]),
@@ -112,6 +113,7 @@ SIGNATURES = {
     "cev_blas_create": (i32, [C.POINTER(P)]),
     "cev_blas_destroy": (i32, [P]),
     "cev_linear": (i32, [P, i32, i32, i64, i64, i64, P, i64, P, i64, C.c_float, P, i64, P, C.c_size_t, P]),
+    "cev_linear_form": (i32, [i32, i64, i64, i64, C.c_size_t, Pi32]),
     "cev_gather_rows": (i32, [i32, i32, i64, i64, P, i64, i64, P, P, i64, P]),
     "cev_table_from_plans": (i32, [i32, Pi32, Pi32, Pi32, i32, Pi32, Pi32, PBlock, i32, Pi32, Pi32, i32, Pi32, Pi32]),
     "cev_table_from_rows": (i32, [i32, i32, i32, i32, Pi32, PBlock, i32]),

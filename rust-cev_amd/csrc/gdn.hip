@@ -1738,11 +1738,14 @@ GdnLayout gdn_layout(const cev_gdn_desc* d) {
 // launch apart, prep works on every chunk at once and the scan on eight
 // 16-column slices of each head at once, which wins for few long rows (one
 // bf16 row of 4096 tokens: 317 against 885).  One chunk is always fused.
-bool use_fused(const GdnArgs& g, bool bf) {
+bool use_fused(const cev_gdn_desc* d) {
+  const bool bf = d->dtype == CEV_BF16;
+  const int64_t conv_dim = 2LL * d->n_k_heads * d->head_k_dim + (int64_t)d->n_v_heads * d->head_v_dim;
+  const int64_t n_chunks = ((int64_t)d->t + kC - 1) / kC;
   // v's buffer offsets are 32-bit; one chunk cannot come near that
-  if (g.n_chunks == 1) return true;
-  if ((int64_t)g.t * g.conv_dim * 2 > INT32_MAX) return false;
-  const double items = (double)g.batch * g.nv, n = g.n_chunks, cus = kConvCus;
+  if (n_chunks == 1) return true;
+  if (d->t * conv_dim * 2 > INT32_MAX) return false;
+  const double items = (double)d->batch * d->n_v_heads, n = (double)n_chunks, cus = kConvCus;
   const double fused = std::ceil(items / cus) * n * (bf ? 14.0 : 20.0);
   const double apart = 15.0 + items * n * (bf ? 0.039 : 0.083) + std::ceil(items * (kD / kW) / cus) * n * (bf ? 3.3 : 3.0);
   return fused < apart;
@@ -1796,6 +1799,14 @@ extern "C" int32_t cev_gdn_desc_init(cev_gdn_desc* d, int32_t dtype, int32_t bat
   d->y_stride_t = vdim;
   d->y_stride_b = vdim * t;
   return check_gdn(d);
+}
+
+extern "C" int32_t cev_gdn_form(const cev_gdn_desc* d, int32_t* fused) {
+  CEV_CHECK_ARG(fused != nullptr, "cev_gdn_form: null output");
+  int32_t rc = check_gdn(d);
+  if (rc) return rc;
+  *fused = d->t > 0 && use_fused(d) ? 1 : 0;
+  return CEV_OK;
 }
 
 extern "C" int32_t cev_gdn_workspace_size(const cev_gdn_desc* d, size_t* bytes) {
@@ -1879,7 +1890,7 @@ extern "C" int32_t cev_gdn_forward(const cev_gdn_desc* d, const void* mixed, con
     launch_conv<__bf16>(g, long_runs, s);
   else
     launch_conv<float>(g, long_runs, s);
-  if (use_fused(g, d->dtype == CEV_BF16)) {
+  if (use_fused(d)) {
     const dim3 grid((unsigned)(g.batch * g.nv));
     if (d->dtype == CEV_BF16)
       hipLaunchKernelGGL(gdn_fused_kernel<__bf16>, grid, dim3(kPrepThreads), 0, s, g);

@@ -655,6 +655,16 @@ extern "C" int32_t cev_linear(cev_blas handle, int32_t dtype, int32_t out_dtype,
                      "hipblasLtMatmul");
 }
 
+extern "C" int32_t cev_linear_form(int32_t dtype, int64_t m, int64_t n, int64_t k, size_t workspace_bytes, int32_t* form) {
+  if (dtype != CEV_F32 && dtype != CEV_BF16) return cev_fail(CEV_ERR_UNSUPPORTED, "cev_linear_form: dtype %d", dtype);
+  CEV_CHECK_ARG(form != nullptr && m >= 0 && n >= 0 && k >= 0, "cev_linear_form: null output or negative size");
+  LinArgs a{};
+  a.m = m, a.n = n, a.k = k;
+  const int parts = dtype == CEV_F32 && m > kRowsSmall && n > 0 && k > 0 ? split_parts(a, workspace_bytes) : 0;
+  *form = m <= kRowsSmall ? 0 : parts > 0 ? parts : -1;
+  return CEV_OK;
+}
+
 extern "C" int32_t cev_gather_rows(int32_t dtype, int32_t out_dtype, int64_t n, int64_t width, const void* table, int64_t ld_table,
                                    int64_t table_rows, const int32_t* ids, void* out, int64_t ld_out, cev_stream stream) {
   if (dtype != CEV_F32 && dtype != CEV_BF16) return cev_fail(CEV_ERR_UNSUPPORTED, "cev_gather_rows: dtype %d", dtype);

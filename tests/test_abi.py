@@ -34,6 +34,34 @@ def test_library_exports_every_header_symbol(cev):
     assert L.cev_abi_version() == 1
 
 
+def test_forms_of_products_and_gdn_calls(cev):
+    """The host queries behind the kernel rules: a product's kernel by its
+    rows, type and workspace, a GDN call's by its rows and length."""
+    L = _abi.lib()
+    form = C.c_int32()
+
+    def linear(dtype, m, n, k, ws=_abi.CEV_LINEAR_WORKSPACE_BYTES):
+        assert L.cev_linear_form(dtype, m, n, k, ws, C.byref(form)) == 0
+        return form.value
+
+    assert linear(CEV_F32, 8, 4096, 2048) == 0 and linear(CEV_BF16, 1, 4096, 2048) == 0
+    assert linear(CEV_F32, 9, 4096, 2048) == -1 and linear(CEV_BF16, 2048, 4096, 2048) == -1
+    assert linear(CEV_F32, 2048, 4096, 2048) == 1 and linear(CEV_F32, 912, 2048, 6144) == 2
+    assert linear(CEV_F32, 912, 2048, 6144, 0) in (-1, 1)  # no room for parts
+    assert L.cev_linear_form(7, 9, 8, 8, 0, C.byref(form)) == CEV_ERR_UNSUPPORTED
+    assert L.cev_linear_form(CEV_F32, 9, 8, 8, 0, None) == CEV_ERR_INVALID
+
+    def gdn(dtype, batch, t):
+        d = _abi.GdnDesc()
+        assert L.cev_gdn_desc_init(C.byref(d), dtype, batch, t, 16, 32, 128, 128, 4, 1e-6) == 0
+        assert L.cev_gdn_form(C.byref(d), C.byref(form)) == 0
+        return form.value
+
+    assert gdn(CEV_BF16, 32, 64) == 1 and gdn(CEV_F32, 1, 1) == 1 and gdn(CEV_BF16, 8, 383) == 1
+    assert gdn(CEV_BF16, 1, 4096) == 0 and gdn(CEV_F32, 1, 65) == 0
+    assert L.cev_gdn_form(None, C.byref(form)) == CEV_ERR_INVALID
+
+
 def test_desc_init_layouts(cev):
     d = cev_hip.attn_desc(CEV_BF16, 32, 8, 128, 4096, 32768)
     assert d.q_stride_t == 32 * 128 and d.q_stride_h == 128

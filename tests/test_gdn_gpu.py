@@ -10,11 +10,13 @@ conv state is a copy and must match bit for bit.  At the 4096-token size the
 oracle runs on a prefix of the sequence, and the split-sequence property
 (T1 then T2 with the carried states == T1 + T2 at once) covers the rest.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import cev_hip
-from cev_hip import configs
+from cev_hip import _abi, configs
 from helpers import to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -25,6 +27,16 @@ BF16_TOL = 2e-2
 
 def _say(msg):
     print(msg, flush=True)
+
+
+def _assert_form(w, fused):
+    """The kernels the library picks for the workload's whole call."""
+    d, form = _abi.GdnDesc(), C.c_int32()
+    L = _abi.lib()
+    _abi.check(L.cev_gdn_desc_init(C.byref(d), cev_hip.CEV_BF16 if w.bf16 else cev_hip.CEV_F32, w.batch, w.t, w.nk, w.nv, w.dk, w.dv,
+                                   w.kernel, w.eps))
+    _abi.check(L.cev_gdn_form(C.byref(d), C.byref(form)))
+    assert form.value == int(fused)
 
 
 def _run_gpu(w, inp, device, conv_in=None, s_in=None, t=None, t0=0):
@@ -400,12 +412,13 @@ def test_conv_on_unaligned_views(gpu, bf16, t):
 
 @pytest.mark.parametrize("bf16", [True, False])
 @pytest.mark.parametrize("batch,t,state", [(1, 1, True), (2, 15, False), (1, 16, True), (3, 17, True), (2, 33, False), (2, 48, True), (1, 49, True),
-                                           (5, 64, True), (9, 65, True), (9, 130, False)])
+                                           (5, 64, True), (25, 65, True), (25, 128, True), (25, 130, False), (25, 192, False), (25, 333, True)])
 def test_fused_rows_vs_oracle(gpu, orc, bf16, batch, t, state):
     """The one-kernel path at the edges of its 16-row tiles and 64-token
-    chunks, with and without a state, against the oracle layer (which works
-    chunk by chunk with explicit inverses)."""
+    chunks, over one to six chunks, with and without a state, against the
+    oracle layer (which works chunk by chunk with explicit inverses)."""
     w = configs.GdnWorkload("gdn-fused", 21 + t, bf16, batch, t, nk=2, nv=4)
+    _assert_form(w, True)
     inp = w.inputs()
     rng = np.random.default_rng(t)
     kw_d, kw_o = {}, {}
@@ -432,6 +445,7 @@ def test_large_finite_values_stay_finite(gpu, orc, bf16, batch, t):
     overflows (they divide to zero): finite results, as the oracle gives them.
     The two large columns are compared relative to their largest value."""
     w = configs.GdnWorkload("gdn-large", 31, bf16, batch, t, nk=2, nv=4)
+    _assert_form(w, True)
     inp = w.inputs()
     s_in = 0.1 * np.random.default_rng(t).standard_normal((batch, 4, 128, 128)).astype(np.float32)
     s_in[0, 0, 3, 7] = 3.4e38

@@ -10,12 +10,14 @@ bf16 budget of the hidden state (2e-2 relative).  The full 28-layer config
 is compared with a fixture the oracle wrote (tests/golden/make_c2_golden.py):
 running the oracle over 1.5e10 FLOP of linear layers takes minutes.
 """
+import ctypes as C
 import os
 
 import numpy as np
 import pytest
 
 from cev_hip import configs
+from cev_hip._abi import CEV_LINEAR_WORKSPACE_BYTES, check, lib
 from helpers import to_np
 
 pytestmark = pytest.mark.gpu
@@ -340,9 +342,9 @@ def test_debias_position_invariant_model_and_invalid_spans(gpu):
     assert np.isnan(got[2, :8]).all() and np.isfinite(got[0, :5]).all() and np.isfinite(got[1, :2]).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(128, 12288, 2048), (700, 2052, 2044), (200, 3000, 6140), (200, 12288, 36), (912, 2048, 6144),
-                                   (1000, 4095, 516), (2050, 4096, 128), (1300, 2048, 2048)])
-def test_split_f32_product(gpu, m, n, k):
+@pytest.mark.parametrize("m,n,k,parts", [(128, 12288, 2048, 2), (700, 2052, 2044, 2), (200, 3000, 6140, 4), (200, 12288, 36, 1),
+                                         (912, 2048, 6144, 2), (1000, 4095, 516, 1), (2050, 4096, 128, 1), (1300, 2048, 2048, 1)])
+def test_split_f32_product(gpu, m, n, k, parts):
     """f32 products on the bf16 matrix cores: remainders of the 128-wide tiles
     and of the 32-deep slices, in one part of k and in several (k = 36: two
     slices, most loads past the end), against f64.
@@ -358,6 +360,9 @@ def test_split_f32_product(gpu, m, n, k):
     import torch
 
     import cev_hip
+    form = C.c_int32()
+    check(lib().cev_linear_form(cev_hip.CEV_F32, m, n, k, CEV_LINEAR_WORKSPACE_BYTES, C.byref(form)))
+    assert form.value == parts
     g = torch.Generator().manual_seed(m + k)
     x, w = torch.randn(m, k, generator=g).to(gpu), torch.randn(n, k, generator=g).to(gpu)
     ld = n + 4 - n % 4 if n % 4 else n
