@@ -69,6 +69,16 @@ def test_token_ids_out_of_range_are_refused():
     assert _i32([1, 2]).dtype == np.int32 and _i32(np.array([3, 4], np.int64)).tolist() == [3, 4]
 
 
+def test_the_library_builds_without_torch():
+    """The default make target compiles no Python module and runs no Python."""
+    import os
+    import subprocess
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "rust-cev_amd")
+    run = subprocess.run(["make", "-n", "-B", "-C", pkg, "PYTHON=/nonexistent"], capture_output=True, text=True)
+    assert run.returncode == 0 and "libcev_hip.so" in run.stdout
+    assert "_cev_calls" not in run.stdout and "nonexistent" not in run.stderr
+
+
 def test_tables_keep_their_blocks(cev):
     """A built table compiles from the builder's array; reading or replacing
     its block list makes the list the table."""
