@@ -82,14 +82,19 @@ class BlockTable:
 
     @blocks.setter
     def blocks(self, value):
-        self._blocks, self._built = list(value), None
+        self._blocks, self._built = value, None
 
     def __len__(self):
         return self._built[1] if self._blocks is None else len(self._blocks)
 
+    def _array(self):
+        """array() for reading: a built table's own array, not a copy."""
+        return self.array() if self._blocks is not None else self._built[0]
+
     def array(self):
+        """The blocks as a ctypes array of the caller's own."""
         if self._blocks is None:
-            return self._built[0]
+            return type(self._built[0]).from_buffer_copy(self._built[0])
         arr = (Block * max(1, len(self.blocks)))()
         for i, b in enumerate(self.blocks):
             arr[i] = b
@@ -230,7 +235,7 @@ class AttnPlan:
 
     def __init__(self, desc: AttnDesc, table: BlockTable, device=None):
         L = lib()
-        arr = table.array()
+        arr = table._array()
         # room for the usual plan (16 bytes a row, a few segments a block);
         # the exact size is asked for only when that was too small
         size = min(1024 + 16 * max(0, int(desc.t)) + 256 * len(table), 1 << 24)

@@ -86,6 +86,8 @@ def test_tables_keep_their_blocks(cev):
     kept = cev_hip.BlockTable.from_plans([(10, 14, 10)], [(0, 3), (0, 5)])[0]
     assert len(tab) == 3 and np.array_equal(tab.to_dense_mask(), kept.to_dense_mask())
     assert [b.as_tuple() for b in tab.blocks] == [tab.array()[i].as_tuple() for i in range(3)]
+    kept.array()[0].q_len = 99  # the caller's copy
+    assert kept.array()[0].q_len != 99
     tab.blocks.pop()
     assert len(tab) == 2 and np.isneginf(tab.to_dense_mask()[-1]).all()
 
