@@ -1624,7 +1624,11 @@ __global__ __launch_bounds__(kPrepThreads) __attribute__((amdgpu_waves_per_eu(2)
         vn[ti] = mma16(a4[e], w, vn[ti]);
       }
     }
-    if (c + 1 < g.n_chunks) load(t0 + kC);
+    if (c + 1 < g.n_chunks) {
+      // this wave's reads of v have returned before the next chunk's v comes over it
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      load(t0 + kC);
+    }
 #pragma unroll
     for (int ti = 0; ti < 4; ++ti) {
       const f32x4 e4 = *(const f32x4*)(L.ecum + 16 * ti + 4 * fq);
