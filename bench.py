@@ -33,15 +33,20 @@ PEAK_TFLOPS = {"bf16": 2516.6, "f32": 157.3}   # dense MFMA at 2.4 GHz
 PEAK_HBM_GBPS = 8000.0
 
 
-# Kernel source each workload's measured traffic depends on.
-TRAFFIC_SOURCES = {"c5gdn": "gdn.hip", "c5gdnrows": "gdn.hip"}
+# Kernel sources each workload's measured traffic depends on (c1 is a small
+# launch: its attention kernel is fan_attn.hip's).
+K2_SOURCES = ("attn_device.h", "packed_attn.hip")
+TRAFFIC_SOURCES = {"c5gdn": ("gdn.hip",), "c5gdnrows": ("gdn.hip",), "c1": K2_SOURCES + ("fan_attn.hip",)}
 
 
-def source_sha16(name: str) -> str:
-    """First 16 hex digits of the SHA-256 of rust-cev_amd/csrc/<name>."""
+def source_sha16(names) -> str:
+    """First 16 hex digits of the SHA-256 of the rust-cev_amd/csrc/<name> files, one after the other."""
     import hashlib
-    with open(os.path.join(ROOT, "rust-cev_amd", "csrc", name), "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()[:16]
+    h = hashlib.sha256()
+    for name in names:
+        with open(os.path.join(ROOT, "rust-cev_amd", "csrc", name), "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()[:16]
 
 
 def traffic_from_profiles(workload: str):
@@ -55,8 +60,7 @@ def traffic_from_profiles(workload: str):
     m = re.search(r"traffic\[%s\]\s*=\s*([0-9.]+)\s+src=([0-9a-f]{16})" % re.escape(workload), open(path).read())
     if not m:
         return None
-    src = TRAFFIC_SOURCES.get(workload, "packed_attn.hip")
-    return float(m.group(1)) if m.group(2) == source_sha16(src) else None
+    return float(m.group(1)) if m.group(2) == source_sha16(TRAFFIC_SOURCES.get(workload, K2_SOURCES)) else None
 
 
 def cpu_model() -> str:
@@ -617,6 +621,8 @@ def main():
     flops = w.useful_flops()
     kernel = {(True, 128): "attn_kernel_pipe<bf16,128>", (True, 256): "attn_kernel_wide<bf16,256>"}.get(
         (w.bf16, w.d), f"attn_kernel_seq<{dtype},{w.d}>")
+    if layer.attn.plan.header()[18]:  # the planner's small-launch form
+        kernel = f"attn_kernel_fan<{dtype},{w.d}>"
     roof = roofline(flops, w.alg_bytes(), k2_ms, dtype, kernel, traffic_from_profiles(w.name))
 
     res = {

@@ -262,7 +262,8 @@ int32_t cev_gdn_form(const cev_gdn_desc* d, int32_t* fused);
  * norm_w are f32 (as GatedDeltaNet::new holds them, qwen35.rs:393-395);
  * s_in / s_out are (B, nv, dk, dv) f32.  conv_in == NULL / s_in == NULL
  * start from zero state (qwen35.rs:426).  conv_out is (B, conv_dim, K-1)
- * contiguous.  Workspace of cev_gdn_workspace_size bytes, 256-byte
+ * contiguous; it may be conv_in's buffer for t <= 4 only (longer rows read
+ * and write the conv state in different workgroups).  Workspace of cev_gdn_workspace_size bytes, 256-byte
  * aligned. */
 int32_t cev_gdn_forward(const cev_gdn_desc* d, const void* mixed, const void* z, const void* b, const void* a, const void* conv_w,
                         const float* neg_a, const float* dt_bias, const float* norm_w, const void* conv_in, const float* s_in, void* y,

@@ -101,12 +101,14 @@ struct Cursor {
 
 // f32: a value as the sum of three bf16 parts (round to nearest each; exact),
 // and six of the nine part products of two such operands, small ones first
-// (the dropped three are below 2^-26).  Six 32x32x16 bf16 MFMAs take 192
-// cycles where the f32 unit takes 512 for the same 16 products; splitting the
-// keys and values costs their wave about as much again, so a sub-tile round
-// went from 5.2 to 4 us (30 x 67-87 rows after 1915 keys 443 -> 390 us).  The
-// error against f64 is smaller (5.1e-7 against 6.0e-7 there): an accumulator
-// is rounded 48 times a sub-tile instead of 64.
+// (of the three dropped ones the two larger are at most 2^-25 of the product
+// each, all three 2^-24).  Six 32x32x16 bf16 MFMAs take 192 cycles where the
+// f32 unit takes 512 for the same 16 products; splitting the keys and values
+// costs their wave about as much again, so a sub-tile round went from 5.2 to
+// 4 us (30 x 67-87 rows after 1915 keys 443 -> 390 us).  The error against 64
+// bits is smaller (5.1e-7 against 6.0e-7 there; 21 % over 44 calls of 1-22
+// blocks after 38-2518 keys, 12-38 % each): an accumulator is rounded 48 times
+// a sub-tile instead of 64.
 namespace split {
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void parts(const float* x, bf16x8* p) {

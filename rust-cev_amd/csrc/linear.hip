@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_rows_kernel(LinArgs a) 
 // that a fragment read touches every bank.
 // What bounds it: a slice takes 3000 clocks a CU where its MFMAs need 1536 and
 // its LDS traffic (195 KB) 1500; 195-202 TFLOP/s of f32 products at 2048 rows
-// (library 146-150).  Tried: one buffer and one slice ahead 134 us at
+// (library 146-151).  Tried: one buffer and one slice ahead 134 us at
 // 200 x 4096 x 2048 (72 now); four waves a tile 89; 64-wide tiles 113 against
 // 95 at 912 x 4096 x 2048; 256 x 128 tiles 4-6 % faster at 2048 rows and half
 // a round short at 912.
@@ -333,9 +333,11 @@ __global__ __launch_bounds__(256) void linear_parts_kernel(const float* ws, LinA
 // times in us: a slice of a 128 x 128 tile takes a CU 1.1, 1.4 when all CUs
 // work (the clock drops), tiles x parts run in rounds of 256, parts are summed
 // by one more pass; the library reaches about 120 TFLOP/s on the f32 unit.
-// The new form has to win by 5 %.  Measured, library -> this (m x n x k):
-//   912 x 4096 x 2048 137 -> 95 us, 912 x 12288 x 2048 355 -> 268,
-//   2048 x 4096 x 2048 261 -> 187, 2048 x 2048 x 6144 346 -> 267;
+// The new form has to win by 5 %.  Measured, library -> this (m x n x k, the
+// same operands again and again; over changing ones both take 2-5 % longer):
+//   912 x 4096 x 2048 119 -> 89 us, 912 x 12288 x 2048 351 -> 258,
+//   912 x 2048 x 6144 174 -> 134 (two parts), 512 x 2048 x 2048 38 -> 34,
+//   2048 x 4096 x 2048 235 -> 176, 2048 x 2048 x 6144 342 -> 255;
 //   200 x 4096 x 2048 (64 tiles) 39 against 72 stays with the library.
 int split_parts(const LinArgs& a, size_t ws_bytes) {
   constexpr int kCus = 256;
