@@ -169,13 +169,15 @@ def test_gdn_conv_widths_vs_oracle(gpu, orc, bf16, kernel):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-def test_gdn_strided_views_vs_oracle(gpu, orc, bf16):
+@pytest.mark.parametrize("t", [70, 40])
+def test_gdn_strided_views_vs_oracle(gpu, orc, bf16, t):
     """z as a column slice of a wider tensor (odd row stride, a view into a
     fused projection output) and y written into such a view: the
-    element-wise norm path.  mixed with rows that are not 16-byte aligned is
+    element-wise norm path of either form.  mixed with rows that are not 16-byte aligned is
     refused (the conv reads 8-element vectors)."""
     import torch
-    w = configs.GdnWorkload("gdn-strided", 13, bf16, 2, 70, nk=2, nv=4)
+    w = configs.GdnWorkload("gdn-strided", 13, bf16, 2, t, nk=2, nv=4)
+    _assert_form(w, t == 40)
     inp = w.inputs()
     dt = torch.bfloat16 if bf16 else torch.float32
     wide = lambda x: torch.cat([torch.zeros(x.shape[:-1] + (1,), dtype=dt, device=gpu), to_dev(np.ascontiguousarray(x), bf16, gpu)], -1)
