@@ -482,6 +482,10 @@ class Blas:
             self._workspace = torch.empty(CEV_LINEAR_WORKSPACE_BYTES, dtype=torch.uint8, device=self._device)
         return self._workspace
 
+    @workspace.setter
+    def workspace(self, buffer):
+        self._workspace = buffer
+
     @classmethod
     def on(cls, device) -> "Blas":
         torch = _torch()
