@@ -16,6 +16,7 @@ host's cores) and, for the default workload, K2 on the HBM-bound
 bidirectional row under c4_shape (both outside the timed steps).
 """
 import argparse
+import ctypes
 import json
 import os
 import re
@@ -261,6 +262,8 @@ def bench_gdn(args, w, dev, traffic_key: str):
         return torch.from_numpy(np.ascontiguousarray(x, np.float32)).to(dev)
 
     layer = cev_hip.GatedDeltaNet(w.batch, w.t, w.nk, w.nv, w.dk, w.dv, w.kernel, w.eps, dtype=mdt, device=dev)
+    fused = ctypes.c_int32()
+    cev_hip._abi.check(cev_hip._abi.lib().cev_gdn_form(ctypes.byref(layer.desc), ctypes.byref(fused)))
     xs = [d(inp[k]) for k in ("mixed", "z", "b", "a", "conv_w")] + [f(inp[k]) for k in ("neg_a", "dt_bias", "norm_w")]
     s_in = conv_in = None
     prefill = None
@@ -322,7 +325,7 @@ def bench_gdn(args, w, dev, traffic_key: str):
                                f"{'bf16' if w.bf16 else 'f32'} inputs, f32 chunk rule",
                    "launch": "hip graph replay" if args.graph else "direct launches",
                    **({"initial_state": prefill} if prefill else {})},
-        "roofline": roofline(w.flops(), alg, layer_ms, "f32", "gdn conv + prep + scan + norm (one forward call)",
+        "roofline": roofline(w.flops(), alg, layer_ms, "f32", f"gdn conv + {'fused kernel' if fused.value else 'prep + scan + norm'} (one forward call)",
                              traffic_from_profiles(traffic_key)),
         "device": device_info().name,
         "settle": dict(SETTLE),
